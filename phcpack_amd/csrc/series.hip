@@ -7,15 +7,17 @@
 //   polynomial eval/diff       GPU_dbl2_poly_evaldiff, Polynomials/dbl2_polynomials_kernels.cu:1577
 // The reference launches one block of deg+1 threads per product and one
 // polynomial per call; here one launch covers a batch of independent
-// instances (one per power-series Newton system or path), the plan holding
-// the monomial structure and coefficients stays resident on the device, and
-// each lane owns one series coefficient of one instance.  The order of the
+// products, and a polynomial takes two, one over all its monomials at a batch
+// of instances (one per power-series Newton system or path), one over its
+// sums; the plan holding the monomial structure and coefficients stays
+// resident on the device.  The order of the
 // multiple-double operations per coefficient is that of the reference host
 // code (CPU_dbl2_product, CPU_dbl2_poly_speel), so results are bit-identical
 // to it.
 #include <hip/hip_runtime.h>
-#include <vector>
+#include <algorithm>
 #include <cstring>
+#include <vector>
 #include "common.hpp"
 #include "mdtypes.hpp"
 #include "../../include/phcmd.h"
@@ -24,27 +26,40 @@ using namespace md;
 
 namespace {
 
+// c ? a : b, limb by limb
+__device__ __forceinline__ double pick_real(bool c, double a, double b) { return c ? a : b; }
+template <int K> __device__ __forceinline__ mdr<K> pick_real(bool c, const mdr<K> &a, const mdr<K> &b) {
+  mdr<K> r;
+#pragma unroll
+  for (int i = 0; i < K; ++i) r.x[i] = c ? a.x[i] : b.x[i];
+  return r;
+}
+
 // number traits: real (K limbs) or complex (2K planes)
 template <int K, bool CPLX> struct Num;
 template <int K> struct Num<K, false> {
   typedef typename RealT<K>::type V;
   static constexpr int P = K;
+  static constexpr bool CX = false;
   __device__ static V load(const double *p, size_t s, size_t j) { return R<K>::load(p, s, j); }
   __device__ static void store(double *p, size_t s, size_t j, const V &v) { R<K>::store(p, s, j, v); }
   __device__ static V mul(const V &a, const V &b) { return md::mul(a, b); }
   __device__ static void mac(V &c, const V &a, const V &b) { c = md::add(c, md::mul(a, b)); }
   __device__ static void inc(V &c, const V &a) { c = md::add(c, a); }
   __device__ static V zero() { return R<K>::zero(); }
+  __device__ static V pick(bool c, const V &a, const V &b) { return pick_real(c, a, b); }
 };
 template <int K> struct Num<K, true> {
   typedef cplx<K> V;
   static constexpr int P = 2 * K;
+  static constexpr bool CX = true;
   __device__ static V load(const double *p, size_t s, size_t j) { return C<K>::load(p, s, j); }
   __device__ static void store(double *p, size_t s, size_t j, const V &v) { C<K>::store(p, s, j, v); }
   __device__ static V mul(const V &a, const V &b) { return C<K>::mul(a, b); }
   __device__ static void mac(V &c, const V &a, const V &b) { C<K>::mac(c, a, b); }
   __device__ static void inc(V &c, const V &a) { c = C<K>::add(c, a); }
   __device__ static V zero() { return C<K>::zero(); }
+  template <class T> __device__ static T pick(bool c, const T &a, const T &b) { return pick_real(c, a, b); }
 };
 
 // ----------------------------------------------------------- elementwise --
@@ -90,132 +105,156 @@ __global__ void __launch_bounds__(256) product_kernel(int D, int nbatch, const d
 
 // ------------------------------------------------ polynomial eval / diff --
 
-// One block holds ipb instances, each owning dpad lanes (lane k = coefficient
-// k).  Monomials are visited in order, as in CPU_dbl2_poly_speel
-// (Polynomials/dbl2_polynomials_host.cpp:13-109); chained products are
-// separated by block barriers because coefficient k of f[j] needs
-// coefficients 0..k of f[j-1], which other lanes produce.
-template <int K, bool CPLX>
-__global__ void __launch_bounds__(256) poly_evaldiff_kernel(int dim, int nbr, int D, const int *__restrict__ nvr,
-                                     const int *__restrict__ idxptr, const int *__restrict__ idx,
-                                     const double *__restrict__ cst, const double *__restrict__ cff,
-                                     int nbatch, const double *__restrict__ input,
-                                     double *__restrict__ output, double *fw, double *bw,
-                                     double *cr, int ipb, int dpad) {
-  typedef Num<K, CPLX> N;
-  typedef typename N::V V;
-  const int sub = threadIdx.x / dpad;
-  const int k = threadIdx.x % dpad;
-  const int b = blockIdx.x * ipb + sub;
-  const bool on = (b < nbatch) && (k < D) && (sub < ipb);
-  const size_t sX = (size_t)nbatch * dim * D;        // input and work plane stride
-  const size_t sO = (size_t)nbatch * (dim + 1) * D;  // output plane stride
-  const size_t sC = (size_t)nbr * D;                 // coefficient plane stride
-  const size_t xb = (size_t)b * dim * D;             // this instance's input / work base
-  const size_t ob = (size_t)b * (dim + 1) * D;       // this instance's output base
-#define XS(r) (xb + (size_t)(r) * D)
-#define OS(r) (ob + (size_t)(r) * D)
-
-  if (on) {
-    N::store(output, sO, OS(dim) + k, N::load(cst, D, k));
-    for (int i = 0; i < dim; ++i) N::store(output, sO, OS(i) + k, N::zero());
+// acc = x*y when first, else acc + x*y, each in the order of N::mul and N::mac
+template <class N>
+__device__ __forceinline__ void mac_or_mul(typename N::V &acc, bool first, const typename N::V &x,
+                                           const typename N::V &y) {
+  if constexpr (N::CX) {
+    const auto re1 = md::mul(x.re, y.re), im1 = md::mul(x.im, y.re);
+    const auto re = N::pick(first, re1, md::add(acc.re, re1));
+    const auto im = N::pick(first, im1, md::add(acc.im, im1));
+    acc.re = md::sub(re, md::mul(x.im, y.im));
+    acc.im = md::add(im, md::mul(x.re, y.im));
+  } else {
+    const auto p = md::mul(x, y);
+    acc = N::pick(first, p, md::add(acc, p));
   }
-  for (int i = 0; i < nbr; ++i) {
-    const int nv = nvr[i];
-    const int *ix = idx + idxptr[i];
-    const size_t co = (size_t)i * D;
-    if (nv == 1) {
-      if (on) {
-        V f = coef_product<N>(input, sX, XS(ix[0]), cff, sC, co, k);
-        V o = N::load(output, sO, OS(dim) + k);
-        N::inc(o, f);
-        N::store(output, sO, OS(dim) + k, o);
-        o = N::load(output, sO, OS(ix[0]) + k);
-        N::inc(o, N::load(cff, sC, co + k));
-        N::store(output, sO, OS(ix[0]) + k, o);
-      }
-    } else if (nv == 2) {
-      if (on) {
-        V f = coef_product<N>(cff, sC, co, input, sX, XS(ix[0]), k);
-        N::store(fw, sX, XS(0) + k, f);
-        V o = N::load(output, sO, OS(ix[1]) + k);
-        N::inc(o, f);
-        N::store(output, sO, OS(ix[1]) + k, o);
-        V g = coef_product<N>(cff, sC, co, input, sX, XS(ix[1]), k);
-        o = N::load(output, sO, OS(ix[0]) + k);
-        N::inc(o, g);
-        N::store(output, sO, OS(ix[0]) + k, o);
-      }
-      __syncthreads();
-      if (on) {
-        V f = coef_product<N>(fw, sX, XS(0), input, sX, XS(ix[1]), k);
-        V o = N::load(output, sO, OS(dim) + k);
-        N::inc(o, f);
-        N::store(output, sO, OS(dim) + k, o);
-      }
-      __syncthreads();
-    } else if (nv > 2) {
-      // forward f[j] and backward b[j] chains advance together
-      if (on) {
-        N::store(fw, sX, XS(0) + k, coef_product<N>(cff, sC, co, input, sX, XS(ix[0]), k));
-        N::store(bw, sX, XS(0) + k,
-                 coef_product<N>(input, sX, XS(ix[nv - 1]), input, sX, XS(ix[nv - 2]), k));
-      }
-      __syncthreads();
-      for (int j = 1; j < nv; ++j) {
-        if (on) {
-          N::store(fw, sX, XS(j) + k,
-                   coef_product<N>(fw, sX, XS(j - 1), input, sX, XS(ix[j]), k));
-          if (j < nv - 2)
-            N::store(bw, sX, XS(j) + k,
-                     coef_product<N>(bw, sX, XS(j - 1), input, sX, XS(ix[nv - 2 - j]), k));
-        }
-        __syncthreads();
-      }
-      V blast;
-      if (on) blast = coef_product<N>(bw, sX, XS(nv - 3), cff, sC, co, k);
-      __syncthreads();
-      if (on) N::store(bw, sX, XS(nv - 3) + k, blast);
-      __syncthreads();
-      if (on) {
-        if (nv == 3) {
-          N::store(cr, sX, XS(0) + k, coef_product<N>(fw, sX, XS(0), input, sX, XS(ix[2]), k));
-        } else {
-          for (int j = 0; j < nv - 3; ++j)
-            N::store(cr, sX, XS(j) + k,
-                     coef_product<N>(fw, sX, XS(j), bw, sX, XS(nv - 4 - j), k));
-          N::store(cr, sX, XS(nv - 3) + k,
-                   coef_product<N>(fw, sX, XS(nv - 3), input, sX, XS(ix[nv - 1]), k));
-        }
-        V o = N::load(output, sO, OS(dim) + k);
-        N::inc(o, N::load(fw, sX, XS(nv - 1) + k));
-        N::store(output, sO, OS(dim) + k, o);
-        o = N::load(output, sO, OS(ix[nv - 1]) + k);
-        N::inc(o, N::load(fw, sX, XS(nv - 2) + k));
-        N::store(output, sO, OS(ix[nv - 1]) + k, o);
-        o = N::load(output, sO, OS(ix[0]) + k);
-        N::inc(o, N::load(bw, sX, XS(nv - 3) + k));
-        N::store(output, sO, OS(ix[0]) + k, o);
-        for (int j = 1; j < nv - 1; ++j) {
-          o = N::load(output, sO, OS(ix[j]) + k);
-          N::inc(o, N::load(cr, sX, XS(j - 1) + k));
-          N::store(output, sO, OS(ix[j]) + k, o);
-        }
-      }
-      __syncthreads();
-    }
-  }
-#undef XS
-#undef OS
 }
 
+// Two truncated products at once by the D lanes of a group: lane k forms
+// coefficient k of x1*y1, then coefficient D-1-k of x2*y2 (when two), so that
+// every lane does D + 1 multiply-adds, where one lane per coefficient of one
+// product leaves half of the lanes idle on average.  The terms of a
+// coefficient keep the order of coef_product.  x1, ...: offsets of the rows
+// in the planar array p (plane stride s).
+template <class N>
+__device__ __forceinline__ void product_pair(const double *p, size_t s, int x1, int y1, int x2, int y2,
+                                             int D, int k, bool two, typename N::V &r1,
+                                             typename N::V &r2) {
+  typename N::V acc = N::zero();
+  const int T = two ? D + 1 : k + 1;
+  for (int it = 0; it < T; ++it) {
+    const bool second = it > k;
+    const int xo = second ? x2 + (it - k - 1) : x1 + it, yo = second ? y2 + (D - it) : y1 + (k - it);
+    mac_or_mul<N>(acc, it == 0 || it == k + 1, N::load(p, s, xo), N::load(p, s, yo));
+    if (it == k) r1 = acc;
+  }
+  r2 = acc;
+}
+
+// The contributions of every monomial at every instance: monomial i's value
+// and its derivatives with respect to idx[idxptr[i]..], in slots idxptr[i]+i
+// (the value) and the nvr[i] slots after it, in contrib [P][nslots][nb][D]
+// for the nb instances b0, b0+1, ... of input [P][nbatch][dim][D].
+//   D lanes (lane k) per monomial and instance; the forward and the backward
+// chain of CPU_dbl2_speel advance together, one product_pair a level, then the
+// cross products in pairs: nv + (nv-2)/2 levels for nv >= 3.  Operands (the
+// variables X, the coefficient C, the chains F and B) are 3 nvmax - 2 rows (at
+// least 2) of the group's work area, in LDS or (LW false) in global memory.
+//   One block walking through all monomials of an instance, the chains in
+// global memory, took 16.4 ms for one double-double polynomial of 560
+// monomials at degree 31 (29 us a monomial, two of the chip's wavefronts
+// busy); monomials are independent, and only the sums over them have an
+// order, which poly_sum_kernel keeps: 75 us for the two kernels.  1021
+// instances of 10 complex quad-double monomials of 4 variables at degree 15:
+// 3.59 -> 0.91 ms (15 TFLOP/s of FP64 operations; the FP64 pipes, about 40
+// TFLOP/s without fused multiply-adds, bound it).
+template <int K, bool CPLX, bool LW>
+__global__ void __launch_bounds__(256) poly_terms_kernel(int dim, int nbr, int D, int nvmax, int rows,
+                                     const int *__restrict__ nvr, const int *__restrict__ idxptr,
+                                     const int *__restrict__ idx, const double *__restrict__ cff,
+                                     int nbatch, int b0, int nb, const double *__restrict__ input,
+                                     double *__restrict__ contrib, size_t sT, double *work, int gpb) {
+  typedef Num<K, CPLX> N;
+  typedef typename N::V V;
+  extern __shared__ double lds[];
+  const int grp = threadIdx.x / D, k = threadIdx.x % D;
+  const size_t gid = (size_t)blockIdx.x * gpb + grp;
+  const bool on = grp < gpb && gid < (size_t)nbr * nb;
+  const int i = on ? (int)(gid / nb) : 0, b = on ? (int)(gid % nb) : 0;
+  const int nv = on ? nvr[i] : 0;
+  const int *ix = idx + idxptr[i];
+  const size_t sX = (size_t)nbatch * dim * D, xb = (size_t)(b0 + b) * dim * D, sC = (size_t)nbr * D;
+  const size_t s = (size_t)rows * D;  // plane stride of the work area
+  double *w = LW ? lds + (size_t)grp * s * N::P : work + gid * s * N::P;
+  auto slot = [&](int j) { return ((size_t)(idxptr[i] + i + j) * nb + b) * D + k; };
+  if (on) {
+    for (int j = 0; j < nv; ++j) N::store(w, s, j * D + k, N::load(input, sX, xb + (size_t)ix[j] * D + k));
+    const V c = N::load(cff, sC, (size_t)i * D + k);
+    N::store(w, s, nv * D + k, c);
+    if (nv == 1) N::store(contrib, sT, slot(1), c);
+  }
+  const int C = nv, F = nv + 1, B = 2 * nv;  // rows: X 0..nv-1, C, F 0..nv-2, B 0..nv-3
+  const int levels = nvmax < 3 ? nvmax : nvmax + (nvmax - 2) / 2;
+  for (int t = 0; t < levels; ++t) {
+    __syncthreads();
+    // the level's products: operand rows, the row to keep a result in and its slot (-1: none)
+    int x1 = -1, y1 = 0, x2 = -1, y2 = 0, d1 = -1, d2 = -1, s1 = -1, s2 = -1;
+    if (nv == 1 && t == 0) {
+      x1 = 0; y1 = C; s1 = 0;
+    } else if (nv == 2 && t == 0) {
+      x1 = C; y1 = 0; d1 = F; s1 = 2;
+      x2 = C; y2 = 1; s2 = 1;
+    } else if (nv == 2 && t == 1) {
+      x1 = F; y1 = 1; s1 = 0;
+    } else if (nv > 2 && t <= nv - 3) {
+      x1 = t ? F + t - 1 : C; y1 = t; d1 = F + t;
+      x2 = t ? B + t - 1 : nv - 1; y2 = nv - 2 - t; d2 = B + t;
+    } else if (nv > 2 && t == nv - 2) {
+      x1 = F + t - 1; y1 = t; d1 = F + t; s1 = nv;
+      x2 = B + t - 1; y2 = C; s2 = 1;
+    } else if (nv > 2 && t == nv - 1) {
+      x1 = F + t - 1; y1 = t; s1 = 0;
+      x2 = F + t - 2; y2 = t; s2 = nv - 1;
+    } else if (nv > 2) {
+      const int j = 2 * (t - nv);
+      if (j < nv - 3) { x1 = F + j; y1 = B + nv - 4 - j; s1 = j + 2; }
+      if (j + 1 < nv - 3) { x2 = F + j + 1; y2 = B + nv - 5 - j; s2 = j + 3; }
+    }
+    if (x1 >= 0) {
+      V r1, r2;
+      const bool two = x2 >= 0;
+      product_pair<N>(w, s, x1 * D, y1 * D, x2 * D, y2 * D, D, k, two, r1, r2);
+      if (d1 >= 0) N::store(w, s, d1 * D + k, r1);
+      if (s1 >= 0) N::store(contrib, sT, slot(s1), r1);
+      if (two) {
+        const int k2 = D - 1 - k;
+        if (d2 >= 0) N::store(w, s, d2 * D + k2, r2);
+        if (s2 >= 0) N::store(contrib, sT, slot(s2) + k2 - k, r2);
+      }
+    }
+  }
+}
+
+// Output row r < dim: the derivative, the sum of its contributions
+// list[lptr[r]..] from zero; row dim: the value, its contributions added to
+// the constant; in the order CPU_dbl2_poly_speel adds them (the monomials'
+// order), one lane per coefficient.  The chain of additions bounds it: the
+// next U contributions are loaded ahead of it.
 template <int K, bool CPLX>
-void launch_poly(int grid, int block, hipStream_t st, int dim, int nbr, int D, const int *nvr,
-                 const int *idxptr, const int *idx, const double *cst, const double *cff,
-                 int nbatch, const double *in, double *out, double *fw, double *bw, double *cr,
-                 int ipb, int dpad) {
-  hipLaunchKernelGGL((poly_evaldiff_kernel<K, CPLX>), dim3(grid), dim3(block), 0, st, dim, nbr,
-                     D, nvr, idxptr, idx, cst, cff, nbatch, in, out, fw, bw, cr, ipb, dpad);
+__global__ void __launch_bounds__(64) poly_sum_kernel(int dim, int D, const int *__restrict__ lptr,
+                                   const int *__restrict__ list, const double *__restrict__ cst,
+                                   int nbatch, int b0, int nb, const double *__restrict__ contrib,
+                                   size_t sT, double *__restrict__ output) {
+  typedef Num<K, CPLX> N;
+  typedef typename N::V V;
+  constexpr int U = N::P <= 2 ? 8 : N::P <= 4 ? 4 : N::P <= 8 ? 2 : 1;
+  const size_t t = (size_t)blockIdx.x * 64 + threadIdx.x, rowlen = (size_t)(dim + 1) * D;
+  if (t >= rowlen * nb) return;
+  const int k = (int)(t % D), r = (int)(t / D % (dim + 1)), b = (int)(t / rowlen);
+  V acc = r == dim ? N::load(cst, D, k) : N::zero();
+  const size_t base = (size_t)b * D + k, step = (size_t)nb * D;
+  const int e1 = lptr[r + 1];
+  int e = lptr[r];
+  for (; e + U <= e1; e += U) {
+    V v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = N::load(contrib, sT, base + list[e + u] * step);
+#pragma unroll
+    for (int u = 0; u < U; ++u) N::inc(acc, v[u]);
+  }
+  for (; e < e1; ++e) N::inc(acc, N::load(contrib, sT, base + list[e] * step));
+  N::store(output, (size_t)nbatch * rowlen, (size_t)(b0 + b) * rowlen + (size_t)r * D + k, acc);
 }
 
 bool valid_k(int K) { return K == 1 || K == 2 || K == 4 || K == 8; }
@@ -226,9 +265,10 @@ bool valid_k(int K) { return K == 1 || K == 2 || K == 4 || K == 8; }
 
 struct phc_poly {
   int K, cplx, dim, nbr, deg;
+  int nvmax = 0, nslots = 0;  // most variables of a monomial; contributions of an instance
   int *d_nvr = nullptr, *d_idxptr = nullptr, *d_idx = nullptr;
+  int *d_lptr = nullptr, *d_list = nullptr;  // per output row, its contributions in order
   double *d_cst = nullptr, *d_cff = nullptr;
-  std::vector<int> nvr;
   double *work = nullptr;
   size_t work_cap = 0;
 };
@@ -286,11 +326,30 @@ int phc_poly_create(phc_poly **plan, int K, int cplx, int dim, int nbr, int deg,
   const int P = cplx ? 2 * K : K, D = deg + 1;
   phc_poly *p = new phc_poly();
   p->K = K; p->cplx = cplx; p->dim = dim; p->nbr = nbr; p->deg = deg;
-  p->nvr.assign(nvr, nvr + nbr);
+  // the contributions of every output row in the order in which
+  // CPU_dbl2_poly_speel adds them: monomial by monomial, two variables as the
+  // second, the first; more as the last, the first, the ones between
+  std::vector<std::vector<int>> rows(dim + 1);
+  for (int i = 0; i < nbr; ++i) {
+    const int nv = nvr[i], *ix = idx + ptr[i], s0 = ptr[i] + i;
+    if (nv > p->nvmax) p->nvmax = nv;
+    rows[dim].push_back(s0);
+    if (nv > 1) rows[ix[nv - 1]].push_back(s0 + nv);
+    rows[ix[0]].push_back(s0 + 1);
+    for (int j = 1; j < nv - 1; ++j) rows[ix[j]].push_back(s0 + 1 + j);
+  }
+  p->nslots = ptr[nbr] + nbr;
+  std::vector<int> lptr(1, 0), list;
+  for (const auto &r : rows) {
+    list.insert(list.end(), r.begin(), r.end());
+    lptr.push_back((int)list.size());
+  }
   const size_t ni = (size_t)std::max(ptr[nbr], 1);
   if (hipMalloc(&p->d_nvr, sizeof(int) * std::max(nbr, 1)) != hipSuccess ||
       hipMalloc(&p->d_idxptr, sizeof(int) * (nbr + 1)) != hipSuccess ||
       hipMalloc(&p->d_idx, sizeof(int) * ni) != hipSuccess ||
+      hipMalloc(&p->d_lptr, sizeof(int) * lptr.size()) != hipSuccess ||
+      hipMalloc(&p->d_list, sizeof(int) * std::max<size_t>(list.size(), 1)) != hipSuccess ||
       hipMalloc(&p->d_cst, sizeof(double) * P * D) != hipSuccess ||
       hipMalloc(&p->d_cff, sizeof(double) * P * std::max(nbr, 1) * D) != hipSuccess) {
     phc_poly_destroy(p);
@@ -301,7 +360,9 @@ int phc_poly_create(phc_poly **plan, int K, int cplx, int dim, int nbr, int deg,
     PHC_HIP(hipMemcpy(p->d_nvr, nvr, sizeof(int) * nbr, hipMemcpyHostToDevice));
     PHC_HIP(hipMemcpy(p->d_idx, idx, sizeof(int) * ptr[nbr], hipMemcpyHostToDevice));
     PHC_HIP(hipMemcpy(p->d_cff, cff, sizeof(double) * P * nbr * D, hipMemcpyHostToDevice));
+    PHC_HIP(hipMemcpy(p->d_list, list.data(), sizeof(int) * list.size(), hipMemcpyHostToDevice));
   }
+  PHC_HIP(hipMemcpy(p->d_lptr, lptr.data(), sizeof(int) * lptr.size(), hipMemcpyHostToDevice));
   PHC_HIP(hipMemcpy(p->d_idxptr, ptr.data(), sizeof(int) * (nbr + 1), hipMemcpyHostToDevice));
   PHC_HIP(hipMemcpy(p->d_cst, cst, sizeof(double) * P * D, hipMemcpyHostToDevice));
   *plan = p;
@@ -310,7 +371,7 @@ int phc_poly_create(phc_poly **plan, int K, int cplx, int dim, int nbr, int deg,
 
 int phc_poly_destroy(phc_poly *p) {
   if (!p) return 0;
-  hipFree(p->d_nvr); hipFree(p->d_idxptr); hipFree(p->d_idx);
+  hipFree(p->d_nvr); hipFree(p->d_idxptr); hipFree(p->d_idx); hipFree(p->d_lptr); hipFree(p->d_list);
   hipFree(p->d_cst); hipFree(p->d_cff); hipFree(p->work);
   delete p;
   return 0;
@@ -322,8 +383,19 @@ int phc_poly_evaldiff(phc_poly *p, int nbatch, const double *input, double *outp
   if (nbatch == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
   const int P = p->cplx ? 2 * p->K : p->K, D = p->deg + 1;
-  const size_t plane = (size_t)nbatch * p->dim * D;
-  const size_t need = 3 * plane * P;
+  // operand rows of a monomial; groups of D lanes per block of 64 (or 1)
+  const int rows = std::max(3 * p->nvmax - 2, 2);
+  const int block = D <= 64 ? 64 : (D + 63) / 64 * 64, gpb = block / D;
+  const size_t group = sizeof(double) * P * rows * D;
+  // LDS while four or more blocks fit a compute unit; beyond that (many
+  // limbs, variables or degrees, where the arithmetic outweighs the loads)
+  // the rows are in global memory and registers alone bound the occupancy
+  const bool lw = group * gpb <= 40 * 1024;
+  // instances per pass: contributions (and rows) up to 256 MiB
+  const size_t inst = sizeof(double) * P * p->nslots * D + (lw ? 0 : group * p->nbr);
+  size_t nbc = inst ? ((size_t)256 << 20) / inst : (size_t)nbatch;
+  nbc = std::min<size_t>(std::max<size_t>(nbc, 1), nbatch);
+  const size_t need = inst / sizeof(double) * nbc;
   if (need > p->work_cap) {
     PHC_HIP(hipStreamSynchronize(st));
     hipFree(p->work);
@@ -332,20 +404,34 @@ int phc_poly_evaldiff(phc_poly *p, int nbatch, const double *input, double *outp
     PHC_HIP(hipMalloc(&p->work, sizeof(double) * need));
     p->work_cap = need;
   }
-  double *fw = p->work, *bw = fw + plane * P, *cr = bw + plane * P;
-  int dpad = 1;
-  while (dpad < D) dpad *= 2;
-  const int block = dpad >= 64 ? dpad : 64;
-  const int ipb = block / dpad;
-  const int grid = (nbatch + ipb - 1) / ipb;
-#define LP(KK, CC) launch_poly<KK, CC>(grid, block, st, p->dim, p->nbr, D, p->d_nvr, p->d_idxptr, p->d_idx, p->d_cst, p->d_cff, nbatch, input, output, fw, bw, cr, ipb, dpad)
-  if (!p->cplx) {
-    if (p->K == 1) LP(1, false); else if (p->K == 2) LP(2, false); else if (p->K == 4) LP(4, false); else LP(8, false);
-  } else {
-    if (p->K == 1) LP(1, true); else if (p->K == 2) LP(2, true); else if (p->K == 4) LP(4, true); else LP(8, true);
-  }
+  for (size_t b0 = 0; b0 < (size_t)nbatch; b0 += nbc) {
+    const int nb = (int)std::min(nbc, (size_t)nbatch - b0);
+    const size_t sT = (size_t)p->nslots * nb * D, ngrp = (size_t)p->nbr * nb;
+    const size_t grid1 = (ngrp + gpb - 1) / gpb, grid2 = ((size_t)nb * (p->dim + 1) * D + 63) / 64;
+    PHC_REQUIRE(grid1 < (1u << 31) && grid2 < (1u << 31), "phc_poly_evaldiff: too many instances");
+#define LP(KK, CC)                                                                               \
+  do {                                                                                           \
+    if (grid1 && lw)                                                                             \
+      hipLaunchKernelGGL((poly_terms_kernel<KK, CC, true>), dim3(grid1), dim3(block),            \
+                         group * gpb, st, p->dim, p->nbr, D, p->nvmax, rows, p->d_nvr,           \
+                         p->d_idxptr, p->d_idx, p->d_cff, nbatch, (int)b0, nb, input, p->work,   \
+                         sT, (double *)nullptr, gpb);                                            \
+    else if (grid1)                                                                              \
+      hipLaunchKernelGGL((poly_terms_kernel<KK, CC, false>), dim3(grid1), dim3(block), 0, st,    \
+                         p->dim, p->nbr, D, p->nvmax, rows, p->d_nvr, p->d_idxptr, p->d_idx,     \
+                         p->d_cff, nbatch, (int)b0, nb, input, p->work, sT, p->work + sT * P,    \
+                         gpb);                                                                   \
+    hipLaunchKernelGGL((poly_sum_kernel<KK, CC>), dim3(grid2), dim3(64), 0, st, p->dim, D,       \
+                       p->d_lptr, p->d_list, p->d_cst, nbatch, (int)b0, nb, p->work, sT, output); \
+  } while (0)
+    if (!p->cplx) {
+      if (p->K == 1) LP(1, false); else if (p->K == 2) LP(2, false); else if (p->K == 4) LP(4, false); else LP(8, false);
+    } else {
+      if (p->K == 1) LP(1, true); else if (p->K == 2) LP(2, true); else if (p->K == 4) LP(4, true); else LP(8, true);
+    }
 #undef LP
-  PHC_HIP(hipGetLastError());
+    PHC_HIP(hipGetLastError());
+  }
   return 0;
 }
 

@@ -106,3 +106,38 @@ def test_poly_evaldiff_batch_vs_oracle(K, cplx):
     out = plan.evaldiff(inp)
     for b in range(nb):
         assert np.array_equal(out[:, b], oracle_poly(K, cplx, nvr, idx, cst, cff, inp[:, b])), b
+
+
+@pytest.mark.parametrize("K,cplx,deg,nb", [(2, 0, 0, 1), (1, 1, 1, 3), (4, 0, 32, 2), (2, 1, 63, 1),
+                                           (2, 0, 64, 3), (8, 1, 40, 1), (4, 1, 6, 130)])
+def test_poly_evaldiff_edges(K, cplx, deg, nb):
+    """One coefficient, groups that do not fill a wavefront or need two, the
+    operand rows in LDS and (K = 8) in global memory, monomials of 1..7
+    variables in one polynomial."""
+    from phcpack_amd.series import PolyPlan
+    rng = np.random.default_rng(900 + 64 * K + deg)
+    dim, nvr = 7, np.array([3, 1, 7, 2, 4, 1, 5, 6, 2], np.int32)
+    supports = [sorted(rng.choice(dim, v, replace=False).tolist()) for v in nvr]
+    idx = np.array([j for s in supports for j in s], np.int32)
+    gen = (lambda s: rand_cmd(rng, K, s)) if cplx else (lambda s: rand_md(rng, K, s))
+    cst, cff, inp = gen((deg + 1,)), gen((len(nvr), deg + 1)), gen((nb, dim, deg + 1))
+    out = PolyPlan(K, cplx, dim, deg, supports, cst, cff).evaldiff(inp)
+    for b in sorted({0, nb // 2, nb - 1}):
+        assert np.array_equal(out[:, b], oracle_poly(K, cplx, nvr, idx, cst, cff, inp[:, b])), b
+
+
+def test_poly_evaldiff_passes():
+    """A batch whose contributions exceed the 256 MiB of one pass (here 62
+    instances), against each instance alone; and a plan without monomials."""
+    from phcpack_amd.series import PolyPlan
+    rng = np.random.default_rng(17)
+    K, dim, deg, nbr, nb = 8, 4, 16, 500, 130
+    supports = [sorted(rng.choice(dim, 3, replace=False).tolist()) for _ in range(nbr)]
+    cst, cff = rand_cmd(rng, K, (deg + 1,)), rand_cmd(rng, K, (nbr, deg + 1))
+    inp = rand_cmd(rng, K, (nb, dim, deg + 1))
+    plan = PolyPlan(K, 1, dim, deg, supports, cst, cff)
+    out = plan.evaldiff(inp)
+    for b in (0, 60, 61, 62, 123, 124, 129):
+        assert np.array_equal(out[:, b:b + 1], plan.evaldiff(np.ascontiguousarray(inp[:, b:b + 1]))), b
+    empty = PolyPlan(K, 1, dim, deg, [], cst, np.zeros((2 * K, 0, deg + 1))).evaldiff(inp[:, :2])
+    assert np.array_equal(empty[:, 1, dim], cst) and not empty[:, :, :dim].any()
