@@ -26,16 +26,19 @@
 //   GPU_cmplx4_bals_qhb                         the GEMM with a split k range
 //     (Newton/dbl4_bals_kernels.cu:602)
 //
-// Every product runs through one complex multiple-double GEMM kernel (32 x 32
-// output tiles, 8-deep k slices staged in LDS, 2 x 2 outputs per lane); long
-// k ranges are split over workgroups whose partial sums are added in slice
-// order by a second kernel.  Results agree with the reference's host
+// The products of quad- and double-double factorizations run on the int8
+// matrix cores (isplit.hpp); small ones, octo-double, Q^H b and what the
+// digits do not cover through one complex multiple-double GEMM kernel (32 x
+// 32 output tiles, 8-deep k slices staged in LDS, 2 x 2 outputs per lane);
+// long k ranges are split over workgroups whose partial sums are added in
+// slice order by a second kernel.  Results agree with the reference's host
 // code to a few units in the last limb (the order of the long sums differs);
 // the tests bound the difference.
 #include <mutex>
 #include <vector>
 
 #include "common.hpp"
+#include "isplit.hpp"
 #include "mdtypes.hpp"
 #include "wave.hpp"
 
@@ -105,15 +108,19 @@ inline int block_rb(int blk) { return (blk >= 3) ? 2 : 1; }
 // the k range over gridDim.z slices, slice s writes its partial sums to
 // part[s][i][j] (plane stride pps) and csum_kernel adds the slices in order.
 // RE: real operands (K planes, no conjugation), real accumulators
+// fa, fb (null: everything): the flags of the operands' digits; only the
+// 64 x 64 blocks that digit_gemm_kernel leaves out are computed
 template <int K, bool CA, bool CB, int RA, int RB, bool RE>
 __global__ void __launch_bounds__(256)
 cgemm_kernel(int M, int N, int KD, int kchunk, Op A, Op B, double *Cp, size_t cps, long c0,
-             long c1, int accumulate, double *part, size_t pps) {
+             long c1, int accumulate, double *part, size_t pps, const int *fa, const int *fb) {
   constexpr int TM = 16 * RA, TN = 16 * RB, PL = RE ? K : 2 * K;
+  static_assert(TM * TKD <= 256 && TN * TKD <= 256);
   __shared__ double As[2 * K][TKD][TM];
   __shared__ double Bs[2 * K][TKD][TN];
   const int t = threadIdx.x, tx = t & 15, ty = t >> 4;
   const int i0 = blockIdx.y * TM, j0 = blockIdx.x * TN;
+  if (fa && !isplit::uncovered(fa, fb, i0, j0)) return;
   const int kb = blockIdx.z * kchunk;
   const int ke = (kb + kchunk) < KD ? (kb + kchunk) : KD;
   Z<K> acc[RA][RB];
@@ -122,8 +129,8 @@ cgemm_kernel(int M, int N, int KD, int kchunk, Op A, Op B, double *Cp, size_t cp
 #pragma unroll
     for (int b = 0; b < RB; ++b) acc[a][b] = C<K>::zero();
   for (int k0 = kb; k0 < ke; k0 += TKD) {
-#pragma unroll
-    for (int e = t; e < TM * TKD; e += 256) {
+    // at most one number of each slice per lane
+    if (const int e = t; e < TM * TKD) {
       int ii, kk;
       if (A.s0 == 1) { ii = e % TM; kk = e / TM; } else { kk = e % TKD; ii = e / TKD; }
       const int gi = i0 + ii, gk = k0 + kk;
@@ -132,8 +139,7 @@ cgemm_kernel(int M, int N, int KD, int kchunk, Op A, Op B, double *Cp, size_t cp
 #pragma unroll
       for (int q = 0; q < PL; ++q) As[q][kk][ii] = in ? A.p[q * A.ps + o] : 0.0;
     }
-#pragma unroll
-    for (int e = t; e < TN * TKD; e += 256) {
+    if (const int e = t; e < TN * TKD) {
       int jj, kk;
       if (B.s1 == 1) { jj = e % TN; kk = e / TN; } else { kk = e % TKD; jj = e / TKD; }
       const int gj = j0 + jj, gk = k0 + kk;
@@ -220,10 +226,10 @@ inline int ksplit(int M, int N, int KD, size_t cap, int TM, int TN, int target) 
 template <int K, bool CA, bool CB, bool RE>
 void launch_gemm(int blk, dim3 grid, hipStream_t st, int M, int N, int KD, int kchunk, Op A,
                  Op B, double *Cp, size_t cps, long c0, long c1, int acc, double *part,
-                 size_t pps) {
+                 size_t pps, const int *fa, const int *fb) {
 #define GEMM(RA_, RB_)                                                                           \
   hipLaunchKernelGGL((cgemm_kernel<K, CA, CB, RA_, RB_, RE>), grid, dim3(256), 0, st, M, N, KD,   \
-                     kchunk, A, B, Cp, cps, c0, c1, acc, part, pps)
+                     kchunk, A, B, Cp, cps, c0, c1, acc, part, pps, fa, fb)
   switch (blk) {
     case 1: GEMM(1, 1); break;
     case 2: GEMM(2, 1); break;
@@ -235,6 +241,23 @@ void launch_gemm(int blk, dim3 grid, hipStream_t st, int M, int N, int KD, int k
 
 // RE: real operands and result (K planes each); the conjugation flags are
 // then ignored
+template <int K, bool RE>
+void launch_gemm_conj(bool ca, bool cb, int blk, dim3 grid, hipStream_t st, int M, int N, int KD,
+                      int kchunk, Op A, Op B, double *Cp, size_t cps, long c0, long c1, int acc,
+                      double *part, size_t pps, const int *fa = nullptr, const int *fb = nullptr) {
+#define LG(CA, CB) \
+  launch_gemm<K, CA, CB, RE>(blk, grid, st, M, N, KD, kchunk, A, B, Cp, cps, c0, c1, acc, part, pps, fa, fb)
+  if constexpr (RE) {
+    LG(false, false);
+  } else {
+    if (!ca && !cb) LG(false, false);
+    else if (ca && !cb) LG(true, false);
+    else if (!ca && cb) LG(false, true);
+    else LG(true, true);
+  }
+#undef LG
+}
+
 template <int K, bool RE = false>
 int cgemm(bool ca, bool cb, int M, int N, int KD, Op A, Op B, double *Cp, size_t cps, long c0,
           long c1, bool accumulate, hipStream_t st, double *part = nullptr, size_t cap = 0,
@@ -247,14 +270,62 @@ int cgemm(bool ca, bool cb, int M, int N, int KD, Op A, Op B, double *Cp, size_t
   dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM, S);
   const int acc = accumulate ? 1 : 0;
   const size_t pps = cap;
-  if (RE) launch_gemm<K, false, false, true>(blk, grid, st, M, N, KD, kchunk, A, B, Cp, cps, c0, c1, acc, part, pps);
-  else if (!ca && !cb) launch_gemm<K, false, false, false>(blk, grid, st, M, N, KD, kchunk, A, B, Cp, cps, c0, c1, acc, part, pps);
-  else if (ca && !cb) launch_gemm<K, true, false, false>(blk, grid, st, M, N, KD, kchunk, A, B, Cp, cps, c0, c1, acc, part, pps);
-  else if (!ca && cb) launch_gemm<K, false, true, false>(blk, grid, st, M, N, KD, kchunk, A, B, Cp, cps, c0, c1, acc, part, pps);
-  else launch_gemm<K, true, true, false>(blk, grid, st, M, N, KD, kchunk, A, B, Cp, cps, c0, c1, acc, part, pps);
+  launch_gemm_conj<K, RE>(ca, cb, blk, grid, st, M, N, KD, kchunk, A, B, Cp, cps, c0, c1, acc, part, pps);
   if (S > 1)
     hipLaunchKernelGGL((csum_kernel<K, RE>), dim3(phc::grid_for((size_t)M * N, 256)), dim3(256), 0, st,
                        M, N, S, part, pps, Cp, cps, c0, c1, acc);
+  PHC_HIP(hipGetLastError());
+  return 0;
+}
+
+// -------------------------------------------- products of digits (int8)
+
+using isplit::Digits;
+using isplit::pad64;
+
+// the digits of the rows of a rows x kd operand, element (r, k) at
+// p[sr*r + sk*k]; conj exchanges im and -im
+template <int K, bool RE>
+int make_digits(Digits &D, const double *p, size_t ps, long sr, long sk, int rows, int kd, bool conj,
+                hipStream_t st) {
+  D.np = RE ? 1 : 3;
+  D.nch = pad64(kd) / 64;
+  hipLaunchKernelGGL((isplit::exponent_kernel<K, RE>), dim3(pad64(rows) / 16), dim3(512), 0, st, p, ps,
+                     sr, sk, rows, kd, D.e, D.flag);
+  hipLaunchKernelGGL((isplit::digit_kernel<K, RE>), dim3(D.nch, pad64(rows) / 16), dim3(256), 0, st, p,
+                     ps, sr, sk, rows, kd, conj ? 1 : 0, D);
+  PHC_HIP(hipGetLastError());
+  return 0;
+}
+
+// C(i, j) = [C(i, j) +] sum_k op(A(i, k)) op(B(k, j)) from the digits Ad of
+// A's rows and Bd of B's columns (three parts when complex, not conjugated
+// unless aconj, bconj say so), and from the operands themselves where the
+// digits do not cover them.  The k range is split while the blocks of 64 x 16
+// outputs do not fill the 256 compute units twice.
+template <int K, bool RE>
+int digit_gemm(bool ca, bool cb, int M, int N, int KD, Digits Ad, bool aconj, Op A, Digits Bd, bool bconj,
+               Op B, double *Cp, size_t cps, long c0, long c1, bool accumulate, hipStream_t st,
+               double *part, size_t cap, GemmCfg cfg) {
+  if (M <= 0 || N <= 0) return 0;
+  const long tiles = (long)(pad64(M) / 64) * ((N + 15) / 16);
+  int S = 1;
+  while (tiles * S * 2 <= 512 && KD / (2 * S) >= 128 && (size_t)M * N * 2 * S <= cap) S *= 2;
+  const int kchunk = pad64((KD + S - 1) / S);
+  const int acc = accumulate ? 1 : 0;
+  constexpr size_t lds = isplit::gemm_lds<K, RE>();
+  PHC_HIP(hipFuncSetAttribute((const void *)isplit::digit_gemm_kernel<K, RE>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL((isplit::digit_gemm_kernel<K, RE>), dim3((N + 15) / 16, pad64(M) / 64, S), dim3(256),
+                     lds, st, M, N, KD, kchunk, Ad, aconj ? 2 : 1, Bd, bconj ? 2 : 1, bconj ? 1 : 2, Cp, cps,
+                     c0, c1, acc, part, cap);
+  const int blk = cfg.block ? cfg.block : default_block<K>();
+  const int TM = 16 * block_ra(blk), TN = 16 * block_rb(blk);
+  launch_gemm_conj<K, RE>(ca, cb, blk, dim3((N + TN - 1) / TN, (M + TM - 1) / TM, S), st, M, N, KD, kchunk,
+                          A, B, Cp, cps, c0, c1, acc, part, cap, Ad.flag, Bd.flag);
+  if (S > 1)
+    hipLaunchKernelGGL((csum_kernel<K, RE>), dim3(phc::grid_for((size_t)M * N, 256)), dim3(256), 0, st,
+                       M, N, S, part, cap, Cp, cps, c0, c1, acc);
   PHC_HIP(hipGetLastError());
   return 0;
 }
@@ -670,9 +741,68 @@ struct phc_baqr {
   const double *gA;
   double *gQ, *gR;
   int greal;  // the captured sequence is the real QR's
+  // digits of the products' operands (split, else null): rows of Y, columns
+  // of Y, of W, of S and of T1, rows of T2, and rows of Q or columns of C, at
+  // most bigrows at a time
+  bool split;
+  Digits Yr, Yc, Wc, Sc, T1c, T2r, big;
+  int bigrows;
 };
 
 namespace {
+
+// the products of tile k with the digits of their operands: every operand is
+// cut once and used by all products it takes part in
+template <int K, bool RE>
+int tile_products(phc_baqr *p, int k, double *Q, double *R, hipStream_t st) {
+  const int m = p->nrows, n = p->ncols, szt = p->szt;
+  const size_t qps = (size_t)m * m, rps = (size_t)m * n;
+  const int rowoff = k * szt, rowdim = m - rowoff, coloff = rowoff + szt, coldim = n - coloff;
+  const Op Yt{p->Y, p->yps, 1, rowdim}, Yc{p->Y, p->yps, rowdim, 1};
+  const Op Wt{p->W, p->yps, 1, rowdim}, Wc{p->W, p->yps, rowdim, 1};
+  // G = Yhat^H Yhat and the S factor
+  if (make_digits<K, RE>(p->Yr, p->Y, p->yps, 1, rowdim, rowdim, szt, false, st) ||
+      make_digits<K, RE>(p->Yc, p->Y, p->yps, rowdim, 1, szt, rowdim, false, st) ||
+      digit_gemm<K, RE>(true, false, szt, szt, rowdim, p->Yc, true, Yc, p->Yc, false, Yt, p->G, p->gps, szt,
+                        1, false, st, p->part, p->pcap, p->cfg))
+    return -1;
+  hipLaunchKernelGGL(s_factor_kernel<K>, dim3(szt), dim3(64), 0, st, p->G, p->gps, p->B, p->S, p->gps, szt);
+  PHC_HIP(hipGetLastError());
+  // W = Yhat S, stored like Y
+  if (make_digits<K, RE>(p->Sc, p->S, p->gps, 1, szt, szt, szt, false, st) ||
+      digit_gemm<K, RE>(false, false, rowdim, szt, szt, p->Yr, false, Yt, p->Sc, false,
+                        Op{p->S, p->gps, szt, 1}, p->W, p->yps, 1, rowdim, false, st, p->part, p->pcap,
+                        p->cfg) ||
+      make_digits<K, RE>(p->Wc, p->W, p->yps, rowdim, 1, szt, rowdim, false, st))
+    return -1;
+  // T1 = What^H C, C += Yhat T1 for the columns of C = R[rowoff.., coloff..]
+  for (int j = 0; j < coldim; j += p->bigrows) {
+    const int nj = coldim - j < p->bigrows ? coldim - j : p->bigrows;
+    double *Cj = R + (size_t)rowoff * n + coloff + j, *T1 = p->T1;
+    const Op Cm{Cj, rps, n, 1}, T1m{T1, p->t1ps, nj, 1};
+    if (make_digits<K, RE>(p->big, Cj, rps, 1, n, nj, rowdim, false, st) ||
+        digit_gemm<K, RE>(true, false, szt, nj, rowdim, p->Wc, true, Wc, p->big, false, Cm, T1, p->t1ps, nj,
+                          1, false, st, p->part, p->pcap, p->cfg) ||
+        make_digits<K, RE>(p->T1c, T1, p->t1ps, 1, nj, nj, szt, false, st) ||
+        digit_gemm<K, RE>(false, false, rowdim, nj, szt, p->Yr, false, Yt, p->T1c, false, T1m, Cj, rps, n, 1,
+                          true, st, p->part, p->pcap, p->cfg))
+      return -1;
+  }
+  // T2 = Q[:, rowoff..] What, Q[:, rowoff..] += T2 Yhat^H for the rows of Q
+  for (int i = 0; i < m; i += p->bigrows) {
+    const int ni = m - i < p->bigrows ? m - i : p->bigrows;
+    double *Qi = Q + (size_t)i * m + rowoff;
+    const Op Qm{Qi, qps, m, 1}, T2m{p->T2, p->t2ps, szt, 1};
+    if (make_digits<K, RE>(p->big, Qi, qps, m, 1, ni, rowdim, false, st) ||
+        digit_gemm<K, RE>(false, false, ni, szt, rowdim, p->big, false, Qm, p->Wc, false, Wt, p->T2, p->t2ps,
+                          szt, 1, false, st, p->part, p->pcap, p->cfg) ||
+        make_digits<K, RE>(p->T2r, p->T2, p->t2ps, szt, 1, ni, szt, false, st) ||
+        digit_gemm<K, RE>(false, true, ni, rowdim, szt, p->T2r, false, T2m, p->Yr, true, Yc, Qi, qps, m, 1,
+                          true, st, p->part, p->pcap, p->cfg))
+      return -1;
+  }
+  return 0;
+}
 
 // RE: A, Q, R are real (K planes); the panel kernels run on the complex
 // workspace with zero imaginary parts, the products on the real planes
@@ -708,6 +838,12 @@ int run_qr(phc_baqr *p, const double *A, double *Q, double *R, hipStream_t st) {
     // Y, W stored as szt rows of length rowdim (row stride rowdim)
     const Op Yt{p->Y, p->yps, 1, rowdim};  // Yhat(i, k) = Y[k][i]
     const Op Yc{p->Y, p->yps, rowdim, 1};  // (k, i) -> Y[k][i]
+    if constexpr (K != 8) {
+      if (p->split) {
+        if (tile_products<K, RE>(p, k, Q, R, st)) return -1;
+        continue;
+      }
+    }
     // G = Yhat^H Yhat
     if (cgemm<K, RE>(true, false, szt, szt, rowdim, Yc, Yt, p->G, p->gps, szt, 1, false, st, p->part,
                  p->pcap, p->cfg)) return -1;
@@ -790,9 +926,40 @@ int tiled_scratch(double **out) {
   return 0;
 }
 
+// the products go through digits where they have enough multiply-adds to pay
+// for cutting the operands and the launches that takes: factorizations of 64 x
+// 64 in tiles of 16 take 5.13 ms by multiply-adds and 4.37 ms by digits
+// (complex quad-double), 1.48 / 1.43 (double-double), 1.03 / 1.11 (real
+// double-double); 96 x 96 in tiles of 32 7.31 / 5.72, 2.05 / 1.70, 1.46 /
+// 1.40; 32 x 32 in tiles of 8 0.76 / 1.02 (double-double)
+bool use_digits(int K, int nrows, int szt) {
+  return K != 8 && (double)nrows * nrows * szt >= 1.5e5;
+}
+
+// digits of the thin operands whole, those of Q and C for at most 128 MiB
+int digit_buffers(phc_baqr *p) {
+  const int m = p->nrows, n = p->ncols, szt = p->szt;
+  auto get = [&](Digits &d, int rows, int k) -> int {
+    const size_t bytes = p->K == 2 ? isplit::digit_bytes<2>(rows, k, 3) : isplit::digit_bytes<4>(rows, k, 3);
+    PHC_HIP(hipMalloc(&d.d, bytes));
+    PHC_HIP(hipMalloc(&d.e, sizeof(int) * 2 * pad64(rows)));
+    d.flag = d.e + pad64(rows);
+    return 0;
+  };
+  const size_t row = p->K == 2 ? isplit::digit_bytes<2>(64, m, 3) : isplit::digit_bytes<4>(64, m, 3);
+  size_t strips = ((size_t)128 << 20) / row;
+  strips = strips < 1 ? 1 : strips;
+  p->bigrows = strips * 64 < (size_t)m ? (int)strips * 64 : m;
+  const int c = n < p->bigrows ? n : p->bigrows, r = m < p->bigrows ? m : p->bigrows;
+  return get(p->Yr, m, szt) || get(p->Yc, szt, m) || get(p->Wc, szt, m) || get(p->Sc, szt, szt) ||
+         get(p->T1c, c, szt) || get(p->T2r, r, szt) || get(p->big, p->bigrows, m);
+}
+
 }  // namespace
 
 extern "C" {
+
+int phc_baqr_destroy(phc_baqr *p);
 
 int phc_baqr_create(phc_baqr **out, int K, int nrows, int ncols, int szt) {
   PHC_REQUIRE(out, "phc_baqr_create: null plan pointer");
@@ -822,6 +989,8 @@ int phc_baqr_create(phc_baqr **out, int K, int nrows, int ncols, int szt) {
   for (int i = 0; i < nb; ++i) *bufs[i] = nullptr;
   p->exec = nullptr;
   p->cap = nullptr;
+  p->split = use_digits(K, nrows, szt);
+  p->Yr = p->Yc = p->Wc = p->Sc = p->T1c = p->T2r = p->big = Digits{nullptr, nullptr, nullptr, 3, 0};
   p->gA = nullptr;
   p->gQ = p->gR = nullptr;
   for (int i = 0; i < nb; ++i) {
@@ -832,9 +1001,14 @@ int phc_baqr_create(phc_baqr **out, int K, int nrows, int ncols, int szt) {
       return -1;
     }
   }
+  if (p->split && digit_buffers(p) != 0) {
+    phc_baqr_destroy(p);
+    phc::set_error("phc_baqr_create: hipMalloc failed");
+    return -1;
+  }
   if (hipStreamCreateWithFlags(&p->cap, hipStreamNonBlocking) != hipSuccess) {
-    for (int j = 0; j < nb; ++j) hipFree(*bufs[j]);
-    delete p;
+    p->cap = nullptr;
+    phc_baqr_destroy(p);
     phc::set_error("phc_baqr_create: hipStreamCreate failed");
     return -1;
   }
@@ -848,6 +1022,10 @@ int phc_baqr_destroy(phc_baqr *p) {
   if (p->cap) hipStreamDestroy(p->cap);
   double *bufs[] = {p->Y, p->W, p->G, p->S, p->T1, p->T2, p->Pc, p->wpart, p->B, p->part};
   for (double *b : bufs) hipFree(b);
+  for (Digits *d : {&p->Yr, &p->Yc, &p->Wc, &p->Sc, &p->T1c, &p->T2r, &p->big}) {
+    hipFree(d->d);
+    hipFree(d->e);
+  }
   delete p;
   return 0;
 }

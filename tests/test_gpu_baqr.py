@@ -216,3 +216,36 @@ def test_real_least_squares_recovers_planted_solution():
     assert np.abs(q.T @ b[0] - y).max() < 1e-12
     x = np.linalg.solve(np.triu(r), y)
     assert np.abs(x - x0).max() < 1e-10
+
+
+
+@pytest.mark.parametrize("K,shape,real,n1", [(4, (140, 128, 64), False, 0), (4, (200, 192, 96), False, 40),
+                                             (4, (150, 128, 64), True, 32), (2, (480, 80, 40), False, 0),
+                                             (2, (384, 128, 64), True, 20), (2, (390, 132, 66), False, 33)])
+def test_qr_by_digit_products(K, shape, real, n1):
+    """The matrix products on the int8 matrix cores (taken at these sizes, not
+    at the smaller ones above): ragged blocks, k beyond one chunk of 64, split
+    sums.  n1 > 0: A = [A11 A12; 0 2^-150 A22] with n1 x n1 A11, whose R keeps
+    the factor 2^-150 in its rows from n1 on: there the columns of W^H C span
+    150 bits, the digits do not cover the small ones, and those blocks go back
+    to the K-limb products; compared relative to their own scale.  Bounds as
+    for the K-limb products."""
+    from oraclelib import oracle_real_blocked_houseqr, rand_md
+    from phcpack_amd.baqr import BlockedQR
+    m, n, szt = shape
+    rng = np.random.default_rng(31 * m + n + K)
+    A = rand_md(rng, K, (m, n)) if real else rand_cmd(rng, K, (m, n))
+    if n1:
+        A[:, n1:, :n1] = 0.0
+        A[:, n1:, n1:] *= 2.0 ** -150
+    qr = BlockedQR(K, m, n, szt)
+    if real:
+        (Q, R), (Qo, Ro) = qr.factor_real(A), oracle_real_blocked_houseqr(K, A, szt, n // szt)
+    else:
+        (Q, R), (Qo, Ro) = qr.factor(A), oracle_blocked_houseqr(K, A, szt, n // szt)
+    tol = QR_UNITS * m * ulps(K)
+    dq, dr = np.abs(md_diff(K, Q, Qo)).max(), np.abs(md_diff(K, R, Ro)).max()
+    ds = np.abs(md_diff(K, R[:, n1:] * 2.0 ** 150, Ro[:, n1:] * 2.0 ** 150)).max() if n1 else 0.0
+    print(f"  K={K} {shape} real={real} n1={n1}: Q {dq / ulps(K):.1f} u, R {dr / ulps(K):.1f} u, "
+          f"small R {ds / ulps(K):.1f} u", flush=True)
+    assert dq < tol and dr < tol * np.sqrt(m) and ds < tol * np.sqrt(m)
