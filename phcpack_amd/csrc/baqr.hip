@@ -5,10 +5,10 @@
 //   reference (Matrices/)                       here
 //   CPU_cmplx4_blocked_houseqr (dbl4_baqr_host.cpp:1206),
 //   GPU_cmplx4_blocked_houseqr (dbl4_baqr_kernels.cu:6197)
-//     per column: house, panel leftRupdate      house_kernel (forms v as well),
-//                                               column_dot_kernel and column_upd_kernel
+//     per column: house, panel leftRupdate      panel_step_kernel: reflector, update and
+//                                               the next column's products in one launch
 //                                               (workgroups per panel column and split
-//                                               of its rows), on a column-major copy
+//                                               of its rows), on column-major copies
 //                                               of the panel; the launches of one
 //                                               factorization replay as a HIP graph
 //     VB_to_W (dbl4_baqr_host.cpp:91)           W = Y S with S upper triangular from
@@ -354,6 +354,9 @@ template <int K> __device__ Z<K> wave_csum(Z<K> s) {
   return C<K>::add(s, bfly_cz<32, K>(s));
 }
 
+// the same for a sum whose imaginary part is zero when RE
+template <int K, bool RE> __device__ Z<K> wave_sum(Z<K> s);
+
 // the butterfly partner's value of a real multiple-double (wave::bfly per limb)
 template <int M, int K> __device__ __forceinline__ T<K> bfly_r(const T<K> &s) {
   T<K> u;
@@ -362,9 +365,20 @@ template <int M, int K> __device__ __forceinline__ T<K> bfly_r(const T<K> &s) {
   return u;
 }
 
-// Out-of-line multiple-double operations for the Householder kernel, whose
-// serial chain (a sum over the column, two square roots, three divisions)
-// runs on a few lanes of one workgroup: one copy of each operation's code
+template <int K, bool RE> __device__ Z<K> wave_sum(Z<K> s) {
+  if constexpr (!RE) return wave_csum<K>(s);
+  s.re = add(s.re, bfly_r<1, K>(s.re));
+  s.re = add(s.re, bfly_r<2, K>(s.re));
+  s.re = add(s.re, bfly_r<4, K>(s.re));
+  s.re = add(s.re, bfly_r<8, K>(s.re));
+  s.re = add(s.re, bfly_r<16, K>(s.re));
+  s.re = add(s.re, bfly_r<32, K>(s.re));
+  return s;
+}
+
+// Out-of-line multiple-double operations for the panel step, whose serial
+// chain (sums, two square roots, divisions) runs on one wavefront of every
+// workgroup: one copy of each operation's code
 // instead of inlined copies at every use (88 KB of straight-line code).
 template <int K> __device__ __noinline__ T<K> nl_add(T<K> a, T<K> b) { return add(a, b); }
 template <int K> __device__ __noinline__ T<K> nl_sub(T<K> a, T<K> b) { return sub(a, b); }
@@ -400,6 +414,210 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+
+constexpr int CW = 256;  // lanes (rows) per workgroup of the panel kernels
+
+// One column of the panel per launch.  The reflector of column L needs, of
+// the columns j >= L of the column-major copy of the panel, H_j = sum_{i>0}
+// conj(R_ij) x_i over the rows below the pivot (x = column L): sigma = H_L,
+// and with v_i = x_i / v0, w_j = beta (conj(R_0j) + H_j / v0).  The step
+// that updates the columns with reflector L forms the H_j of the next pivot
+// column from the rows that it has just updated, so a column costs one
+// launch; it reads the panel from one copy and writes the other, since every
+// block forms the new values of the next pivot column's rows as well.
+//   Before, the Householder vector, the products w_j and the update were
+// three launches of 28 + 12 + 9 us a column (1024 x 1024 complex quad-double),
+// each waiting for the previous one's sums.  What bounds the step is the
+// chain of dependent quad-double operations: two roots on two lanes, two
+// divisions, the butterflies of the sums.
+//
+//   Workgroup (c, s): column j = colidx + c, rows of split s (CW of them, one
+// per lane, counted from the pivot row).  hpart[s][c]: the partial sums of H
+// that the previous step left in ns_in splits; hout likewise.
+//   Wavefront 0, the scalars as CPU_cmplx2_factors_house forms them
+// (Matrices/dbl2_factorizations.cpp:441-533): 16 lanes each add up H of the
+// pivot column, of column c and of the next pivot column; nrm = sqrt(|x0|^2 +
+// sigma) on even lanes and r0 = |x0| on odd ones in one root; mu = nrm / r0;
+// v0 = x0 - mu x0 (re on even, im on odd lanes); beta = 2 |v0|^2 / (sigma +
+// |v0|^2) and conj(v0) / |v0|^2 in one division; sigma = 0: beta = 0, v_i =
+// x_i.  RE (real data, zero imaginary parts; CPU_dbl4_factors_house,
+// Matrices/dbl4_factorizations.cpp:541-626): mu = sqrt(x0^2 + sigma), v0 =
+// x0 - mu when the leading limb of x0 is <= 0, else -sigma/(x0 + mu), beta =
+// 2 v0^2 / (sigma + v0^2), v_i = x_i / v0.
+//   Sums are in tree order (the reference's are sequential): results agree to
+// a few units in the last limb.
+template <int K, bool RE>
+__global__ void __launch_bounds__(CW)
+panel_step_kernel(const double *Pin, double *Pout, size_t pps, int m, int rowoff, int colidx, int nrows,
+                  int L, double *Y, size_t yps, int rowdim, double *Bv, int szt, const double *hpart,
+                  int ns_in, double *hout, size_t hps) {
+  __shared__ Z<K> part[CW / 64];
+  __shared__ Z<K> sinv, sown, snext;  // 1/v0 (RE: v0), w_j, w of the next pivot column
+  __shared__ int sflag;
+  const int t = threadIdx.x, c = blockIdx.x, n = nrows - colidx, i = blockIdx.y * CW + t;
+  const bool in = i < n, last = L + 1 == szt;
+  const size_t col = (size_t)(colidx - rowoff) * m + colidx;  // x_i at col + i, R_ij at + c m
+  // this lane's row of the pivot column, of column c and of the next one
+  Z<K> xi = C<K>::zero(), ri = C<K>::zero(), ni = C<K>::zero();
+  if (in) {
+    xi = C<K>::load(Pin, pps, col + i);
+    ri = C<K>::load(Pin, pps, col + (size_t)c * m + i);
+    if (c > 1) ni = C<K>::load(Pin, pps, col + m + i);
+  }
+  if (c == 0 && blockIdx.y == 0)
+    for (int q = t; q < L; q += CW) C<K>::store(Y, yps, (size_t)L * rowdim + q, C<K>::zero());
+  if (t < 64) {
+    const int g = t >> 4, u = t & 15;
+    const int cg = g == 0 ? 0 : g == 1 ? c : last ? 0 : 1;
+    const Z<K> x0 = C<K>::load(Pin, pps, col), r0g = C<K>::load(Pin, pps, col + (size_t)cg * m);
+    Z<K> h = C<K>::zero();
+    if (u < ns_in) h = C<K>::load(hpart, hps, (size_t)u * szt + L + cg);
+    for (int q = u + 16; q < ns_in; q += 16) {
+      const Z<K> hq = C<K>::load(hpart, hps, (size_t)q * szt + L + cg);
+      h.re = nl_add<K>(h.re, hq.re);
+      h.im = nl_add<K>(h.im, hq.im);
+    }
+    auto stage = [&](const Z<K> &o) { h.re = nl_add<K>(h.re, o.re); h.im = nl_add<K>(h.im, o.im); };
+    if (ns_in > 1) stage(bfly_cz<1, K>(h));
+    if (ns_in > 2) stage(bfly_cz<2, K>(h));
+    if (ns_in > 4) stage(bfly_cz<4, K>(h));
+    if (ns_in > 8) stage(bfly_cz<8, K>(h));
+    const T<K> sigma = lane_r<K>(h.re, 0), sq0 = nl_norm2<K>(x0);
+    bool szero = true;
+#pragma unroll
+    for (int q = 0; q < K; ++q) szero = szero && (sigma.x[q] == 0.0);
+    T<K> beta = R<K>::zero();
+    Z<K> inv = C<K>::zero();
+    if (!szero) {
+      if constexpr (RE) {
+        const T<K> mu = nl_sqrt<K>(nl_add<K>(sq0, sigma));
+        T<K> v0;
+        if (R<K>::hi(x0.re) <= 0.0) v0 = nl_sub<K>(x0.re, mu);
+        else v0 = neg(nl_div<K>(sigma, nl_add<K>(x0.re, mu)));
+        // even lanes: beta / 2, odd lanes: 1 / v0
+        const T<K> v0p2 = nl_mul<K>(v0, v0), den = nl_add<K>(sigma, v0p2);
+        const T<K> qt = (t & 1) ? nl_div<K>(R<K>::from(1.0), v0) : nl_div<K>(v0p2, den);
+        beta = mul_d(lane_r<K>(qt, 0), 2.0);
+        inv.re = lane_r<K>(qt, 1);
+        if (t == 0) sinv.re = v0;
+      } else {
+        T<K> rt = sq0;
+        if ((t & 1) == 0) rt = nl_add<K>(sq0, sigma);
+        rt = nl_sqrt<K>(rt);
+        const T<K> nrm = lane_r<K>(rt, 0), r0 = lane_r<K>(rt, 1);
+        bool rz = true;
+#pragma unroll
+        for (int q = 0; q < K; ++q) rz = rz && (r0.x[q] == 0.0);
+        // even lanes: v0.re, odd lanes: v0.im
+        const T<K> xc = (t & 1) ? x0.im : x0.re;
+        T<K> vc;
+        if (rz) vc = (t & 1) ? R<K>::zero() : neg(nrm);
+        else vc = nl_sub<K>(xc, nl_mul<K>(nl_div<K>(nrm, r0), xc));
+        const T<K> vsq = nl_mul<K>(vc, vc);
+        const T<K> sqrv0 = nl_add<K>(lane_r<K>(vsq, 0), lane_r<K>(vsq, 1));
+        // lanes 0 and 1: conj(v0) / |v0|^2, lanes 2 and 3: beta / 2
+        T<K> num = vc, den = sqrv0;
+        if (t & 2) {
+          num = sqrv0;
+          den = nl_add<K>(sigma, sqrv0);
+        }
+        const T<K> qt = nl_div<K>(num, den);
+        beta = mul_d(lane_r<K>(qt, 2), 2.0);
+        inv.re = lane_r<K>(qt, 0);
+        inv.im = neg(lane_r<K>(qt, 1));
+        if (t == 0) sinv = inv;
+      }
+    }
+    // w = beta (conj(R_0) + H inv) of the group's column
+    Z<K> w;
+    if constexpr (RE) {
+      w.re = nl_mul<K>(beta, nl_add<K>(r0g.re, nl_mul<K>(h.re, inv.re)));
+      w.im = R<K>::zero();
+    } else {
+      const T<K> hre = nl_sub<K>(nl_mul<K>(h.re, inv.re), nl_mul<K>(h.im, inv.im));
+      const T<K> him = nl_add<K>(nl_mul<K>(h.im, inv.re), nl_mul<K>(h.re, inv.im));
+      w.re = nl_mul<K>(beta, nl_add<K>(r0g.re, hre));
+      w.im = nl_mul<K>(beta, nl_sub<K>(him, r0g.im));
+    }
+    if (t == 0) {
+      sflag = szero ? 1 : 0;
+      if (c == 0 && blockIdx.y == 0) R<K>::store(Bv, szt, L, beta);
+    }
+    if (t == 16) sown = w;
+    if (t == 32) snext = w;
+  }
+  __syncthreads();
+  Z<K> v;
+  if (i == 0) {
+    v = C<K>::from(1.0, 0.0);
+  } else if (sflag) {
+    v = xi;
+  } else if constexpr (RE) {
+    v.re = nl_div<K>(xi.re, sinv.re);
+    v.im = R<K>::zero();
+  } else {
+    const Z<K> inv = sinv;
+    v.re = sub(mul(xi.re, inv.re), mul(xi.im, inv.im));
+    v.im = add(mul(xi.im, inv.re), mul(xi.re, inv.im));
+  }
+  // r - v conj(w)
+  auto update = [&](const Z<K> &r, const Z<K> &w) {
+    Z<K> o;
+    if constexpr (RE) {
+      o.re = sub(r.re, mul(v.re, w.re));
+      o.im = R<K>::zero();
+    } else {
+      o.re = sub(r.re, add(mul(v.re, w.re), mul(v.im, w.im)));
+      o.im = sub(r.im, sub(mul(v.im, w.re), mul(v.re, w.im)));
+    }
+    return o;
+  };
+  ri = update(ri, sown);
+  if (in) {
+    C<K>::store(Pout, pps, col + (size_t)c * m + i, ri);
+    if (c == 0) C<K>::store(Y, yps, (size_t)L * rowdim + L + i, v);
+  }
+  if (c == 0) return;
+  // H of the next pivot column: the rows below its pivot, row 1 here
+  ni = c == 1 ? ri : update(ni, snext);
+  Z<K> s = C<K>::zero();
+  if (in && i > 1) {
+    if constexpr (RE) {
+      s.re = mul(ri.re, ni.re);
+    } else {
+      s.re = add(mul(ri.re, ni.re), mul(ri.im, ni.im));
+      s.im = sub(mul(ri.re, ni.im), mul(ri.im, ni.re));
+    }
+  }
+  s = wave_sum<K, RE>(s);
+  if ((t & 63) == 0) part[t >> 6] = s;
+  __syncthreads();
+  if (t == 0)
+    C<K>::store(hout, hps, (size_t)blockIdx.y * szt + L + c,
+                C<K>::add(C<K>::add(part[0], part[1]), C<K>::add(part[2], part[3])));
+}
+
+// H of the first pivot column (the panel as it comes), as the steps leave it
+template <int K, bool RE>
+__global__ void __launch_bounds__(CW)
+panel_first_kernel(const double *Pin, size_t pps, int m, int rowoff, int nrows, int szt, double *hout,
+                   size_t hps) {
+  __shared__ Z<K> part[CW / 64];
+  const int t = threadIdx.x, c = blockIdx.x, i = blockIdx.y * CW + t;
+  Z<K> s = C<K>::zero();
+  if (i > 0 && i < nrows - rowoff)
+    cmac<K, true, false>(s, C<K>::load(Pin, pps, (size_t)c * m + rowoff + i),
+                         C<K>::load(Pin, pps, rowoff + i));
+  s = wave_sum<K, RE>(s);
+  if ((t & 63) == 0) part[t >> 6] = s;
+  __syncthreads();
+  if (t == 0)
+    C<K>::store(hout, hps, (size_t)blockIdx.y * szt + c,
+                C<K>::add(C<K>::add(part[0], part[1]), C<K>::add(part[2], part[3])));
+}
+
+// ---- the octo-double panel: three launches a column.  One step in one kernel
+// would keep five octo-double complex numbers per lane live and spill 1.5 KB.
 
 constexpr int HW = 1024;  // lanes of the Householder kernel
 
@@ -545,8 +763,6 @@ house_kernel(const double *Pc, size_t pps, int m, int rowoff, int colidx, int nr
   for (int i = ir + stride; i < n; i += stride) C<K>::store(yl, yps, i, vof(x(i)));
 }
 
-constexpr int CW = 256;  // lanes (rows) per workgroup of the column kernels
-
 // The panel part of the reference's leftRupdate (Matrices/dbl4_baqr_host.cpp:
 // 357) for the columns j = colidx + c of the column-major copy Pc, with the
 // rows split over workgroups of CW lanes (one row per lane):
@@ -596,57 +812,71 @@ column_upd_kernel(double *Pc, size_t pps, int m, int rowoff, int colidx, int nro
   C<K>::store(col, pps, i, r);
 }
 
-// the panel columns rowoff..rowoff+szt-1 of R (rows rowoff..m-1) to and from
-// the column-major copy Pc
+// the panel columns rowoff..rowoff+szt-1 of R (rows rowoff..m-1) to the
+// column-major copy P0, or back: step L reads copy L mod 2 and writes the
+// other one from row L on, so the last to write row i of column c is step
+// min(i, c)
 template <int K, bool RE>
 __global__ void panel_copy_kernel(double *Rm, size_t rps, int ld, int m, int rowoff, int szt,
-                                  double *Pc, size_t pps, int to_panel) {
+                                  double *P0, double *P1, size_t pps, int to_panel) {
   const size_t rows = (size_t)(m - rowoff), tot = rows * szt;
   for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < tot;
        e += (size_t)gridDim.x * blockDim.x) {
-    const int c = (int)(e / rows), i = rowoff + (int)(e % rows);
-    const size_t re = (size_t)i * ld + rowoff + c, pe = (size_t)c * m + i;
+    const int c = (int)(e / rows), i = (int)(e % rows);
+    const size_t re = (size_t)(rowoff + i) * ld + rowoff + c, pe = (size_t)c * m + rowoff + i;
     if (to_panel)
-      C<K>::store(Pc, pps, pe, Acc<K, RE>::load(Rm, rps, re));
+      C<K>::store(P0, pps, pe, Acc<K, RE>::load(Rm, rps, re));
     else
-      Acc<K, RE>::store(Rm, rps, re, C<K>::load(Pc, pps, pe));
+      Acc<K, RE>::store(Rm, rps, re, C<K>::load(((i < c ? i : c) & 1) ? P0 : P1, pps, pe));
   }
 }
 
 // S (szt x szt, upper triangular, row-major) with W = Y S:
-// S[j][j] = -B_j, S[m][j] = -B_j sum_{k=m}^{j-1} S[m][k] G[k][j]; one
-// wavefront per row m (kept in LDS), lanes split the sum over k
+// S[j][j] = -B_j, S[m][j] = -B_j sum_{k=m}^{j-1} S[m][k] G[k][j], in the
+// order of k.  One wavefront per row m, lanes own the columns j = l, l + 64,
+// ... and add S[m][k] G[k][j] as soon as S[m][k] is known: a step of the chain
+// is a product by B_k and a multiply-add, where a sum over lanes for every j
+// took a multiply-add, six butterfly additions and a product (1085 us for 128
+// complex quad-double columns).
 template <int K>
 __global__ void __launch_bounds__(64)
 s_factor_kernel(const double *G, size_t gps, const double *Bv, double *S, size_t sps, int szt) {
-  __shared__ double row[2 * K][256];
   const int m = blockIdx.x, l = threadIdx.x;
-  for (int j = 0; j < szt; ++j) {
-    Z<K> s = C<K>::zero();
-    if (j > m) {
-      for (int k = m + l; k < j; k += 64)
-        s = C<K>::add(s, C<K>::mul(C<K>::load(&row[0][0], 256, k),
-                                    C<K>::load(G, gps, (size_t)k * szt + j)));
-      s = wave_csum<K>(s);
+  constexpr int NJ = 2;  // szt <= 128
+  Z<K> acc[NJ];
+#pragma unroll
+  for (int q = 0; q < NJ; ++q) acc[q] = C<K>::zero();
+  for (int k = m; k < szt; ++k) {
+    const T<K> b = neg(R<K>::load(Bv, szt, k));
+    const Z<K> a = (k >> 6) ? acc[1] : acc[0];
+    Z<K> v;
+    if (k == m) {
+      v.re = b;
+      v.im = R<K>::zero();
+    } else {
+      v.re = mul(b, lane_r<K>(a.re, k & 63));
+      v.im = mul(b, lane_r<K>(a.im, k & 63));
     }
-    if (l == 0) {
-      const T<K> b = neg(R<K>::load(Bv, szt, j));
-      Z<K> v;
-      if (j < m) v = C<K>::zero();
-      else if (j == m) { v.re = b; v.im = R<K>::zero(); }
-      else { v.re = mul(b, s.re); v.im = mul(b, s.im); }
-      C<K>::store(&row[0][0], 256, j, v);
+    if (l == (k & 63)) C<K>::store(S, sps, (size_t)m * szt + k, v);
+#pragma unroll
+    for (int q = 0; q < NJ; ++q) {
+      const int j = l + 64 * q;
+      if (j > k && j < szt)
+        acc[q] = C<K>::add(acc[q], C<K>::mul(v, C<K>::load(G, gps, (size_t)k * szt + j)));
     }
-    __syncthreads();
   }
-  for (int j = l; j < szt; j += 64) C<K>::store(S, sps, (size_t)m * szt + j, C<K>::load(&row[0][0], 256, j));
+  for (int j = l; j < m; j += 64) C<K>::store(S, sps, (size_t)m * szt + j, C<K>::zero());
 }
 
 // ------------------------------------------------------- tiled solver
 
 // inverse of the diagonal tiles of U (dim x dim): one wavefront per column j
-// of tile t, x = T^{-1} e_j by back substitution with the sums over k split
-// across lanes; x kept in LDS, written to inv[t][szt][szt]
+// of tile t, x = T^{-1} e_j by back substitution: lanes own rows r and subtract
+// U[r][i] x_i as soon as x_i is known.  The reciprocals of the diagonal are
+// formed first, a lane each (octo-double: divided by at each step), so a step
+// of the chain is a product and a multiply-add; a sum over lanes and a
+// division per row took 2.0 ms for tiles of 128 in complex quad-double.  The
+// right-hand sides turn into x in LDS, and x is written to inv[t][szt][szt].
 template <int K>
 __global__ void __launch_bounds__(256)
 tile_inverse_kernel(const double *U, size_t ups, int dim, int szt, int ntiles, double *inv,
@@ -658,21 +888,34 @@ tile_inverse_kernel(const double *U, size_t ups, int dim, int szt, int ntiles, d
   const int tile = id / szt, j = id % szt, off = tile * szt;
   double *x = &xs[wv][0][0];
   const size_t ib = (size_t)tile * szt * szt;
-  for (int i = szt - 1; i >= 0; --i) {
-    Z<K> v = C<K>::zero();
-    if (i <= j) {
-      Z<K> s = C<K>::zero();
-      for (int k = i + 1 + l; k <= j; k += 64)
-        s = C<K>::add(s, C<K>::mul(C<K>::load(U, ups, (size_t)(off + i) * dim + off + k),
-                                    C<K>::load(x, 256, k)));
-      s = wave_csum<K>(s);
-      v = C<K>::sub(i == j ? C<K>::from(1.0, 0.0) : C<K>::zero(), s);
-      v = C<K>::div(v, C<K>::load(U, ups, (size_t)(off + i) * dim + off + i));
+  auto u = [&](int r, int c) { return C<K>::load(U, ups, (size_t)(off + r) * dim + off + c); };
+  constexpr int NR = K == 8 ? 1 : 4;  // szt <= 256
+  Z<K> rc[NR];
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    const int r = l + 64 * q;
+    if (K < 8 && r <= j) rc[q] = C<K>::div(C<K>::from(1.0, 0.0), u(r, r));
+  }
+  for (int r = l; r < szt; r += 64) C<K>::store(x, 256, r, C<K>::from(r == j ? 1.0 : 0.0, 0.0));
+  wave_sync();
+  for (int i = j; i >= 0; --i) {
+    Z<K> v = C<K>::load(x, 256, i);
+    if constexpr (K == 8) {
+      v = C<K>::div(v, u(i, i));
+    } else {
+      Z<K> a = rc[0], b;
+#pragma unroll
+      for (int q = 1; q < NR; ++q)
+        if ((i >> 6) == q) a = rc[q];
+      b.re = lane_r<K>(a.re, i & 63);
+      b.im = lane_r<K>(a.im, i & 63);
+      v = C<K>::mul(v, b);
     }
-    if (l == 0) C<K>::store(x, 256, i, v);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync();
+    if (l == (i & 63)) C<K>::store(x, 256, i, v);
+    for (int r = l; r < i; r += 64)
+      C<K>::store(x, 256, r, C<K>::sub(C<K>::load(x, 256, r), C<K>::mul(u(r, i), v)));
+    wave_sync();
   }
   for (int i = l; i < szt; i += 64) C<K>::store(inv, ips, ib + (size_t)i * szt + j, C<K>::load(x, 256, i));
 }
@@ -733,8 +976,8 @@ __global__ void zero_kernel(double *p, size_t n) {
 struct phc_baqr {
   int K, nrows, ncols, szt, nbt;
   GemmCfg cfg;  // GEMM launch configuration of the plan's products
-  double *Y, *W, *G, *S, *T1, *T2, *Pc, *wpart, *B, *part;
-  size_t yps, gps, t1ps, t2ps, pps, wpps, pcap;
+  double *Y, *W, *G, *S, *T1, *T2, *Pc, *hpart, *B, *part;
+  size_t yps, gps, t1ps, t2ps, pps, hps, pcap;
   // the launch sequence of one factorization, captured for the last (A, Q, R)
   hipStream_t cap;
   hipGraphExec_t exec;
@@ -818,22 +1061,37 @@ int run_qr(phc_baqr *p, const double *A, double *Q, double *R, hipStream_t st) {
   PHC_HIP(hipGetLastError());
   for (int k = 0; k < p->nbt; ++k) {
     const int rowoff = k * szt, rowdim = m - rowoff, endcol = (k + 1) * szt;
-    hipLaunchKernelGGL((panel_copy_kernel<K, RE>), dim3(phc::grid_for((size_t)rowdim * szt, 256)),
-                       dim3(256), 0, st, R, rps, n, m, rowoff, szt, p->Pc, p->pps, 1);
-    for (int L = 0; L < szt; ++L) {
-      const int colidx = rowoff + L, ncol = endcol - colidx;
-      const int nr = m - colidx, ns = (nr + CW - 1) / CW;
-      const int hwv = (nr - 1 + 63) / 64, hw = 64 * (hwv < 1 ? 1 : hwv < HW / 64 ? hwv : HW / 64);
-      hipLaunchKernelGGL((house_kernel<K, RE>), dim3(1), dim3(hw), 0, st, p->Pc, p->pps, m, rowoff,
-                         colidx, m, L, p->Y, p->yps, rowdim, p->B, szt);
-      hipLaunchKernelGGL(column_dot_kernel<K>, dim3(ncol, ns), dim3(CW), 0, st, p->Pc, p->pps, m,
-                         rowoff, colidx, m, p->Y, p->yps, rowdim, L, p->wpart, p->wpps, szt);
-      hipLaunchKernelGGL(column_upd_kernel<K>, dim3(ncol, ns), dim3(CW), 0, st, p->Pc, p->pps, m,
-                         rowoff, colidx, m, p->Y, p->yps, rowdim, L, p->wpart, p->wpps, ns, p->B,
-                         szt);
+    const int copies = phc::grid_for((size_t)rowdim * szt, 256);
+    double *const Pc[2] = {p->Pc, K == 8 ? p->Pc : p->Pc + 2 * (size_t)K * p->pps};
+    double *const hp[2] = {p->hpart, p->hpart + 2 * (size_t)K * p->hps};
+    hipLaunchKernelGGL((panel_copy_kernel<K, RE>), dim3(copies), dim3(256), 0, st, R, rps, n, m, rowoff,
+                       szt, Pc[0], Pc[1], p->pps, 1);
+    if constexpr (K == 8) {
+      for (int L = 0; L < szt; ++L) {
+        const int colidx = rowoff + L, ncol = endcol - colidx;
+        const int nr = m - colidx, ns = (nr + CW - 1) / CW;
+        const int hwv = (nr - 1 + 63) / 64, hw = 64 * (hwv < 1 ? 1 : hwv < HW / 64 ? hwv : HW / 64);
+        hipLaunchKernelGGL((house_kernel<K, RE>), dim3(1), dim3(hw), 0, st, Pc[0], p->pps, m, rowoff,
+                           colidx, m, L, p->Y, p->yps, rowdim, p->B, szt);
+        hipLaunchKernelGGL(column_dot_kernel<K>, dim3(ncol, ns), dim3(CW), 0, st, Pc[0], p->pps, m,
+                           rowoff, colidx, m, p->Y, p->yps, rowdim, L, hp[0], p->hps, szt);
+        hipLaunchKernelGGL(column_upd_kernel<K>, dim3(ncol, ns), dim3(CW), 0, st, Pc[0], p->pps, m,
+                           rowoff, colidx, m, p->Y, p->yps, rowdim, L, hp[0], p->hps, ns, p->B, szt);
+      }
+    } else {
+      int ns = (rowdim + CW - 1) / CW;
+      hipLaunchKernelGGL((panel_first_kernel<K, RE>), dim3(szt, ns), dim3(CW), 0, st, Pc[0], p->pps, m,
+                         rowoff, m, szt, hp[0], p->hps);
+      for (int L = 0; L < szt; ++L) {
+        const int colidx = rowoff + L, in = L & 1, ns_in = ns;
+        ns = (m - colidx + CW - 1) / CW;
+        hipLaunchKernelGGL((panel_step_kernel<K, RE>), dim3(szt - L, ns), dim3(CW), 0, st, Pc[in],
+                           Pc[in ^ 1], p->pps, m, rowoff, colidx, m, L, p->Y, p->yps, rowdim, p->B, szt,
+                           hp[in], ns_in, hp[in ^ 1], p->hps);
+      }
     }
-    hipLaunchKernelGGL((panel_copy_kernel<K, RE>), dim3(phc::grid_for((size_t)rowdim * szt, 256)),
-                       dim3(256), 0, st, R, rps, n, m, rowoff, szt, p->Pc, p->pps, 0);
+    hipLaunchKernelGGL((panel_copy_kernel<K, RE>), dim3(copies), dim3(256), 0, st, R, rps, n, m, rowoff,
+                       szt, Pc[0], Pc[1], p->pps, 0);
     PHC_HIP(hipGetLastError());
     // Y, W stored as szt rows of length rowdim (row stride rowdim)
     const Op Yt{p->Y, p->yps, 1, rowdim};  // Yhat(i, k) = Y[k][i]
@@ -974,16 +1232,16 @@ int phc_baqr_create(phc_baqr **out, int K, int nrows, int ncols, int szt) {
   p->t1ps = (size_t)szt * ncols;
   p->t2ps = (size_t)nrows * szt;
   p->pps = (size_t)szt * nrows;
-  p->wpps = (size_t)szt * ((nrows + CW - 1) / CW);
+  p->hps = (size_t)szt * ((nrows + CW - 1) / CW);
   // split-k partial sums: up to 8 slices of the largest thin product, and
   // the Q^H b products (nrows x 1 in up to 32 slices)
   p->pcap = (size_t)nrows * szt * 8;
   if ((size_t)nrows * 32 > p->pcap) p->pcap = (size_t)nrows * 32;
   const size_t z = sizeof(double) * 2 * K;
   double **bufs[] = {&p->Y,  &p->W,     &p->G, &p->S,   &p->T1,
-                     &p->T2, &p->Pc, &p->wpart, &p->B, &p->part};
+                     &p->T2, &p->Pc, &p->hpart, &p->B, &p->part};
   const size_t sizes[] = {z * p->yps, z * p->yps, z * p->gps, z * p->gps, z * p->t1ps,
-                          z * p->t2ps, z * p->pps, z * p->wpps, sizeof(double) * K * szt,
+                          z * p->t2ps, 2 * z * p->pps, 2 * z * p->hps, sizeof(double) * K * szt,
                           z * p->pcap};
   const int nb = 10;
   for (int i = 0; i < nb; ++i) *bufs[i] = nullptr;
@@ -1020,7 +1278,7 @@ int phc_baqr_destroy(phc_baqr *p) {
   if (!p) return 0;
   if (p->exec) hipGraphExecDestroy(p->exec);
   if (p->cap) hipStreamDestroy(p->cap);
-  double *bufs[] = {p->Y, p->W, p->G, p->S, p->T1, p->T2, p->Pc, p->wpart, p->B, p->part};
+  double *bufs[] = {p->Y, p->W, p->G, p->S, p->T1, p->T2, p->Pc, p->hpart, p->B, p->part};
   for (double *b : bufs) hipFree(b);
   for (Digits *d : {&p->Yr, &p->Yc, &p->Wc, &p->Sc, &p->T1c, &p->T2r, &p->big}) {
     hipFree(d->d);
