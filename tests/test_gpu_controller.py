@@ -26,6 +26,35 @@ def test_mlp_forward_and_grad_match_numpy():
     assert np.allclose(g, g_ref, rtol=1e-3, atol=1e-5 * np.abs(g_ref).max())
 
 
+@pytest.mark.parametrize("F,H,C,B", [(16, 64, 6, 1), (16, 64, 12, 17), (3, 64, 16, 4099), (16, 64, 1, 16390),
+                                     (20, 32, 5, 70), (16, 48, 6, 33)])
+def test_mlp_shapes_match_numpy(F, H, C, B):
+    """One row, ragged tiles of 16 rows, more rows than one pass of the blocks
+    takes, fewer inputs and all 16 candidates in the one-kernel path; shapes
+    beyond it layer by layer; candidates out of range count for nothing.
+    FP32 sums of up to B terms: relative error below 2^-24 B^(1/2) of the
+    terms' size, far below the bounds."""
+    from phcpack_amd._lib import DeviceArray, check, load
+    from phcpack_amd.controller import forward_np, grad_np
+    rng = np.random.default_rng(B + C)
+    w = (rng.standard_normal(F * H + H + H * H + H + H * C + C) * 0.2).astype(np.float32)
+    X = rng.standard_normal((B, F)).astype(np.float32)
+    cand, y = rng.integers(0, C, B).astype(np.int32), rng.integers(0, 2, B).astype(np.float32)
+    d = [DeviceArray.from_host(a) for a in (w, X, cand, y)]
+    dl, dg, ds = DeviceArray((B, C), np.float32), DeviceArray((len(w),), np.float32), DeviceArray((1,), np.float32)
+    check(load().phc_mlp_forward(F, H, C, d[0].ptr, B, d[1].ptr, dl.ptr, None))
+    O, _ = forward_np(w, X.astype(np.float64), F, H, C)
+    assert np.allclose(dl.to_host(), O, rtol=1e-4, atol=1e-5)
+    check(load().phc_mlp_grad(F, H, C, d[0].ptr, B, d[1].ptr, d[2].ptr, d[3].ptr, dg.ptr, ds.ptr, None))
+    g, loss = grad_np(w, X.astype(np.float64), cand, y.astype(np.float64), F, H, C)
+    assert abs(float(ds.to_host()[0]) - loss) <= 1e-5 * loss
+    # a hidden unit within rounding of zero may be on one side only: 1/B of its gradient
+    assert np.allclose(dg.to_host(), g, rtol=1e-3, atol=(1e-5 + 1.0 / B / 64) * np.abs(g).max())
+    out = DeviceArray.from_host(np.full(B, C, np.int32))
+    check(load().phc_mlp_grad(F, H, C, d[0].ptr, B, d[1].ptr, out.ptr, d[3].ptr, dg.ptr, ds.ptr, None))
+    assert not dg.to_host().any() and float(ds.to_host()[0]) == 0.0
+
+
 def test_mlp_training_reduces_loss():
     from phcpack_amd.controller import MULTS, NFEAT, StepController
     rng = np.random.default_rng(1)
