@@ -46,6 +46,17 @@ __device__ __forceinline__ void wsync() {
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 
+// The lanes that work on one system together: one wavefront (several of them
+// in a block, each with its own system), or TW > 1 wavefronts, the whole block.
+template <int TW> struct Team {
+  static constexpr int N = 64 * TW;
+  __device__ static __forceinline__ int id() { return TW == 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x; }
+  __device__ static __forceinline__ void sync() {
+    if constexpr (TW == 1) wsync();
+    else __syncthreads();
+  }
+};
+
 __device__ __forceinline__ double wave_fmax(double v) { return wave::max64(v); }
 
 constexpr size_t LDS_LIMIT = 160 * 1024;
@@ -126,6 +137,15 @@ template <int K> __device__ __forceinline__ bool all_zero(const mdr<K> &a) {
 __device__ __forceinline__ double limb(double a, int) { return a; }
 template <int K> __device__ __forceinline__ double limb(const mdr<K> &a, int i) { return a.x[i]; }
 
+// c ? a : b, limb by limb
+__device__ __forceinline__ double choose(bool c, double a, double b) { return c ? a : b; }
+template <int K> __device__ __forceinline__ mdr<K> choose(bool c, const mdr<K> &a, const mdr<K> &b) {
+  mdr<K> r;
+#pragma unroll
+  for (int i = 0; i < K; ++i) r.x[i] = c ? a.x[i] : b.x[i];
+  return r;
+}
+
 // carve a planar array of m numbers out of LDS
 template <int K, bool CX = false> __device__ Arr<K, CX> carve(double *&p, int m) {
   Arr<K, CX> a{p, m};
@@ -135,8 +155,10 @@ template <int K, bool CX = false> __device__ Arr<K, CX> carve(double *&p, int m)
 
 // largest |leading limb| of v[0..n-1], as CPU_dbl_onenorm computes it
 // (Newton/dbl_onenorms_host.cpp:9-17): NaN when v[0] is NaN, later NaNs
-// skipped.  Uniform over the wavefront; every lane must call it.
-template <int K, bool CX = false> __device__ double maxnorm(const Arr<K, CX> &v, int off, int n) {
+// skipped.  Uniform over the team (every wavefront takes all n); every lane
+// must call it.
+template <int K, bool CX = false, class A = Arr<K, CX>>
+__device__ double maxnorm(const A &v, int off, int n) {
   const int l = lane_id();
   double r = 0.0, v0 = 0.0;
   for (int i = l; i < n; i += 64) {
@@ -160,15 +182,15 @@ template <int K, bool CX = false> struct LinWork {
 // Q R = A for the n x n matrix given by the accessor a(r, c)
 // (CPU_dbl2_factors_houseqr with CPU_dbl2_factors_house, leftRupdate and
 // rightQupdate, Matrices/dbl2_factorizations.cpp:374-440, 534-566, 629-660)
-template <int K, class A> __device__ void houseqr(int n, const A &a, const LinWork<K> &w) {
+template <int K, int TW, class A> __device__ void houseqr(int n, const A &a, const LinWork<K> &w) {
   typedef typename RealT<K>::type T;
-  const int l = lane_id();
-  for (int t = l; t < n * n; t += 64) {
+  const int l = Team<TW>::id();
+  for (int t = l; t < n * n; t += Team<TW>::N) {
     const int i = t / n, j = t % n;
     w.q.st(t, R<K>::from(i == j ? 1.0 : 0.0));
     w.r.st(t, a(i, j));
   }
-  wsync();
+  Team<TW>::sync();
   for (int k = 0; k < n; ++k) {
     const int m = n - k;
     // Householder vector of x = R[k..n-1][k]: sigma, mu, v0, beta in lane 0
@@ -200,12 +222,12 @@ template <int K, class A> __device__ void houseqr(int n, const A &a, const LinWo
         w.sc.st(1, v0);
       }
     }
-    wsync();
+    Team<TW>::sync();
     {
       const T v0 = w.sc.ld(1);
       const bool szero = R<K>::hi(w.sc.ld(2)) != 0.0;
       // v[i] = x[i] / v0 (x[i] unchanged when sigma = 0), v[0] = 1
-      for (int i = l; i < m; i += 64) {
+      for (int i = l; i < m; i += Team<TW>::N) {
         if (i == 0) w.v.st(0, R<K>::from(1.0));
         else {
           const T xi = w.r.ld((k + i) * n + k);
@@ -213,56 +235,56 @@ template <int K, class A> __device__ void houseqr(int n, const A &a, const LinWo
         }
       }
     }
-    wsync();
+    Team<TW>::sync();
     const T beta = w.sc.ld(0);
     // w1[j-k] = beta * sum_i R[i][j] v[i-k]
-    for (int j = k + l; j < n; j += 64) {
+    for (int j = k + l; j < n; j += Team<TW>::N) {
       T s = R<K>::zero();
       for (int i = k; i < n; ++i) s = add(s, mul(w.r.ld(i * n + j), w.v.ld(i - k)));
       w.w1.st(j - k, mul(beta, s));
     }
     // w2[i] = beta * sum_{j>=k} Q[i][j] v[j-k]
-    for (int i = l; i < n; i += 64) {
+    for (int i = l; i < n; i += Team<TW>::N) {
       T s = R<K>::zero();
       for (int j = k; j < n; ++j) s = add(s, mul(w.q.ld(i * n + j), w.v.ld(j - k)));
       w.w2.st(i, mul(beta, s));
     }
-    wsync();
+    Team<TW>::sync();
     // R[i][j] -= v[i-k] w1[j-k];  Q[i][j] -= w2[i] v[j-k]
-    for (int t = l; t < m * m; t += 64) {
+    for (int t = l; t < m * m; t += Team<TW>::N) {
       const int i = k + t / m, j = k + t % m;
       w.r.st(i * n + j, sub(w.r.ld(i * n + j), mul(w.v.ld(i - k), w.w1.ld(j - k))));
     }
-    for (int t = l; t < n * m; t += 64) {
+    for (int t = l; t < n * m; t += Team<TW>::N) {
       const int i = t / m, j = k + t % m;
       w.q.st(i * n + j, sub(w.q.ld(i * n + j), mul(w.w2.ld(i), w.v.ld(j - k))));
     }
-    wsync();
+    Team<TW>::sync();
   }
 }
 
 // x = R^{-1} Q^T b (CPU_dbl2_factors_qrbs and _backward): b = bv[bo..],
 // x = xv[xo..]; b and x may be the same row.
-template <int K>
-__device__ void qrbs(int n, const LinWork<K> &w, const Arr<K> &bv, int bo, const Arr<K> &xv,
+template <int K, int TW, class BV>
+__device__ void qrbs(int n, const LinWork<K> &w, const BV &bv, int bo, const Arr<K> &xv,
                      int xo) {
   typedef typename RealT<K>::type T;
-  const int l = lane_id();
-  for (int i = l; i < n; i += 64) {
+  const int l = Team<TW>::id();
+  for (int i = l; i < n; i += Team<TW>::N) {
     T s = R<K>::zero();
     for (int j = 0; j < n; ++j) s = add(s, mul(w.q.ld(j * n + i), bv.ld(bo + j)));
     w.wrk.st(i, s);
   }
-  wsync();
-  for (int i = l; i < n; i += 64) xv.st(xo + i, w.wrk.ld(i));
-  wsync();
+  Team<TW>::sync();
+  for (int i = l; i < n; i += Team<TW>::N) xv.st(xo + i, w.wrk.ld(i));
+  Team<TW>::sync();
   // column sweep: row i receives the terms j = n-1 .. i+1 in that order
   for (int j = n - 1; j >= 0; --j) {
-    if (l == (j & 63)) xv.st(xo + j, div(xv.ld(xo + j), w.r.ld(j * n + j)));
-    wsync();
+    if (l == j) xv.st(xo + j, div(xv.ld(xo + j), w.r.ld(j * n + j)));
+    Team<TW>::sync();
     const T xj = xv.ld(xo + j);
-    for (int i = l; i < j; i += 64) xv.st(xo + i, sub(xv.ld(xo + i), mul(w.r.ld(i * n + j), xj)));
-    wsync();
+    for (int i = l; i < j; i += Team<TW>::N) xv.st(xo + i, sub(xv.ld(xo + i), mul(w.r.ld(i * n + j), xj)));
+    Team<TW>::sync();
   }
 }
 
@@ -273,16 +295,16 @@ __device__ void qrbs(int n, const LinWork<K> &w, const Arr<K> &bv, int bo, const
 // beta = 2 |v0|^2 / (sigma + |v0|^2), 1/v0 = conj(v0) / |v0|^2), the lanes
 // v_i = x_i / v0, then w1 = beta R^H v, w2 = beta Q v and the rank-one
 // updates R -= v w1^H, Q -= w2 v^H, every entry in the reference's order.
-template <int K, class A> __device__ void cx_houseqr(int n, const A &a, const LinWork<K, true> &w) {
+template <int K, int TW, class A> __device__ void cx_houseqr(int n, const A &a, const LinWork<K, true> &w) {
   typedef typename RealT<K>::type T;
   typedef cplx<K> Z;
-  const int l = lane_id();
-  for (int t = l; t < n * n; t += 64) {
+  const int l = Team<TW>::id();
+  for (int t = l; t < n * n; t += Team<TW>::N) {
     const int i = t / n, j = t % n;
     w.q.st(t, C<K>::from(i == j ? 1.0 : 0.0, 0.0));
     w.r.st(t, a(i, j));
   }
-  wsync();
+  Team<TW>::sync();
   for (int k = 0; k < n; ++k) {
     const int m = n - k;
     if (l == 0) {
@@ -329,11 +351,11 @@ template <int K, class A> __device__ void cx_houseqr(int n, const A &a, const Li
         w.sc.st(1, inv);
       }
     }
-    wsync();
+    Team<TW>::sync();
     {
       const Z inv = w.sc.ld(1);
       const bool szero = R<K>::hi(w.sc.ld(2).im) != 0.0;
-      for (int i = l; i < m; i += 64) {
+      for (int i = l; i < m; i += Team<TW>::N) {
         if (i == 0) {
           w.v.st(0, C<K>::from(1.0, 0.0));
         } else {
@@ -351,10 +373,10 @@ template <int K, class A> __device__ void cx_houseqr(int n, const A &a, const Li
         }
       }
     }
-    wsync();
+    Team<TW>::sync();
     const T beta = w.sc.ld(0).re;
     // w1[j-k] = beta * sum_i conj(R[i][j]) v[i-k]
-    for (int j = k + l; j < n; j += 64) {
+    for (int j = k + l; j < n; j += Team<TW>::N) {
       Z s = C<K>::zero();
       for (int i = k; i < n; ++i) {
         const Z r = w.r.ld(i * n + j), v = w.v.ld(i - k);
@@ -370,7 +392,7 @@ template <int K, class A> __device__ void cx_houseqr(int n, const A &a, const Li
       w.w1.st(j - k, s);
     }
     // w2[i] = beta * sum_{j>=k} Q[i][j] v[j-k]
-    for (int i = l; i < n; i += 64) {
+    for (int i = l; i < n; i += Team<TW>::N) {
       Z s = C<K>::zero();
       for (int j = k; j < n; ++j) {
         const Z q = w.q.ld(i * n + j), v = w.v.ld(j - k);
@@ -385,9 +407,9 @@ template <int K, class A> __device__ void cx_houseqr(int n, const A &a, const Li
       s.im = mul(beta, s.im);
       w.w2.st(i, s);
     }
-    wsync();
+    Team<TW>::sync();
     // R[i][j] -= v[i-k] conj(w1[j-k]);  Q[i][j] -= w2[i] conj(v[j-k])
-    for (int t = l; t < m * m; t += 64) {
+    for (int t = l; t < m * m; t += Team<TW>::N) {
       const int i = k + t / m, j = k + t % m;
       const Z v = w.v.ld(i - k), x = w.w1.ld(j - k);
       Z r = w.r.ld(i * n + j);
@@ -399,7 +421,7 @@ template <int K, class A> __device__ void cx_houseqr(int n, const A &a, const Li
       r.im = sub(r.im, zim);
       w.r.st(i * n + j, r);
     }
-    for (int t = l; t < n * m; t += 64) {
+    for (int t = l; t < n * m; t += Team<TW>::N) {
       const int i = t / m, j = k + t % m;
       const Z x = w.w2.ld(i), v = w.v.ld(j - k);
       Z q = w.q.ld(i * n + j);
@@ -411,19 +433,19 @@ template <int K, class A> __device__ void cx_houseqr(int n, const A &a, const Li
       q.im = sub(q.im, zim);
       w.q.st(i * n + j, q);
     }
-    wsync();
+    Team<TW>::sync();
   }
 }
 
 // x = R^{-1} Q^H b (CPU_cmplx2_factors_qrbs and _backward, Matrices/
 // dbl2_factorizations.cpp:842-879, 142-200): b = bv[bo..], x = xv[xo..]
-template <int K>
-__device__ void cx_qrbs(int n, const LinWork<K, true> &w, const Arr<K, true> &bv, int bo,
+template <int K, int TW, class BV>
+__device__ void cx_qrbs(int n, const LinWork<K, true> &w, const BV &bv, int bo,
                         const Arr<K, true> &xv, int xo) {
   typedef typename RealT<K>::type T;
   typedef cplx<K> Z;
-  const int l = lane_id();
-  for (int i = l; i < n; i += 64) {
+  const int l = Team<TW>::id();
+  for (int i = l; i < n; i += Team<TW>::N) {
     Z s = C<K>::zero();
     for (int j = 0; j < n; ++j) {
       const Z q = w.q.ld(j * n + i), b = bv.ld(bo + j);
@@ -434,11 +456,11 @@ __device__ void cx_qrbs(int n, const LinWork<K, true> &w, const Arr<K, true> &bv
     }
     w.wrk.st(i, s);
   }
-  wsync();
-  for (int i = l; i < n; i += 64) xv.st(xo + i, w.wrk.ld(i));
-  wsync();
+  Team<TW>::sync();
+  for (int i = l; i < n; i += Team<TW>::N) xv.st(xo + i, w.wrk.ld(i));
+  Team<TW>::sync();
   for (int j = n - 1; j >= 0; --j) {
-    if (l == (j & 63)) {
+    if (l == j) {
       const Z u = w.r.ld(j * n + j), x = xv.ld(xo + j);
       const T den = add(mul(u.re, u.re), mul(u.im, u.im));
       const T a1re = div(u.re, den), a1im = neg(div(u.im, den));
@@ -447,9 +469,9 @@ __device__ void cx_qrbs(int n, const LinWork<K, true> &w, const Arr<K, true> &bv
       y.im = add(mul(x.im, a1re), mul(x.re, a1im));
       xv.st(xo + j, y);
     }
-    wsync();
+    Team<TW>::sync();
     const Z xj = xv.ld(xo + j);
-    for (int i = l; i < j; i += 64) {
+    for (int i = l; i < j; i += Team<TW>::N) {
       const Z u = w.r.ld(i * n + j);
       Z y = xv.ld(xo + i);
       const T a1re = mul(u.re, xj.re), a1im = mul(u.im, xj.im);
@@ -460,20 +482,20 @@ __device__ void cx_qrbs(int n, const LinWork<K, true> &w, const Arr<K, true> &bv
       y.im = sub(y.im, a2im);
       xv.st(xo + i, y);
     }
-    wsync();
+    Team<TW>::sync();
   }
 }
 
 // the real or complex factorization and solve
-template <int K, bool CX, class A> __device__ void any_houseqr(int n, const A &a, const LinWork<K, CX> &w) {
-  if constexpr (CX) cx_houseqr<K>(n, a, w);
-  else houseqr<K>(n, a, w);
+template <int K, bool CX, int TW, class A>
+__device__ void any_houseqr(int n, const A &a, const LinWork<K, CX> &w) {
+  if constexpr (CX) cx_houseqr<K, TW>(n, a, w);
+  else houseqr<K, TW>(n, a, w);
 }
-template <int K, bool CX>
-__device__ void any_qrbs(int n, const LinWork<K, CX> &w, const Arr<K, CX> &bv, int bo,
-                         const Arr<K, CX> &xv, int xo) {
-  if constexpr (CX) cx_qrbs<K>(n, w, bv, bo, xv, xo);
-  else qrbs<K>(n, w, bv, bo, xv, xo);
+template <int K, bool CX, int TW, class BV>
+__device__ void any_qrbs(int n, const LinWork<K, CX> &w, const BV &bv, int bo, const Arr<K, CX> &xv, int xo) {
+  if constexpr (CX) cx_qrbs<K, TW>(n, w, bv, bo, xv, xo);
+  else qrbs<K, TW>(n, w, bv, bo, xv, xo);
 }
 
 struct Flags {
@@ -483,20 +505,20 @@ struct Flags {
 // lower block-triangular Toeplitz solve sum_{j<=k} A_j x_{k-j} = b_k
 // (CPU_dbl2_qrbs_solve with _head and _tail); mat(j, r, c) = A_j[r][c];
 // rhs and sol rows k at offsets k*n.  Uniform control flow.
-template <int K, bool CX, class M>
-__device__ void qrbs_solve(int n, int degp1, int tailidx, const M &mat, const Arr<K, CX> &rhs,
+template <int K, bool CX, int TW, class M, class BV>
+__device__ void qrbs_solve(int n, int degp1, int tailidx, const M &mat, const BV &rhs,
                            const Arr<K, CX> &sol, const LinWork<K, CX> &w, Flags &f) {
   typedef typename NT<K, CX>::V T;
-  const int l = lane_id();
+  const int l = Team<TW>::id();
   const double thr = threshold<K>();
   if (!(f.noqr && !f.zeroQ)) {
     const double nrm = maxnorm<K, CX>(rhs, 0, n);
     const bool small = (K == 1) ? (nrm + 1.0 == 1.0) : (nrm < thr);
     if (small) f.noqr = f.zeroQ ? 0 : 1;
     if (!f.noqr) {
-      any_houseqr<K, CX>(n, [&](int r, int c) { return mat(0, r, c); }, w);
+      any_houseqr<K, CX, TW>(n, [&](int r, int c) { return mat(0, r, c); }, w);
       f.zeroQ = 0;
-      any_qrbs<K, CX>(n, w, rhs, 0, sol, 0);
+      any_qrbs<K, CX, TW>(n, w, rhs, 0, sol, 0);
     }
   }
   if (degp1 > 1) {
@@ -508,25 +530,25 @@ __device__ void qrbs_solve(int n, int degp1, int tailidx, const M &mat, const Ar
         ++skipup;
       } else {
         const int npair = (degp1 - i) * n;
-        for (int t = l; t < npair; t += 64) {
+        for (int t = l; t < npair; t += Team<TW>::N) {
           const int j = i + t / n, k = t % n;
           T b = rhs.ld(j * n + k);
           for (int L = 0; L < n; ++L) b = NT<K, CX>::msub(b, mat(j - i + 1, k, L), sol.ld((i - 1) * n + L));
           rhs.st(j * n + k, b);
         }
       }
-      wsync();
+      Team<TW>::sync();
       const double nrm = maxnorm<K, CX>(rhs, i * n, n);
       if (nrm < thr || nrm > 1.0e+99) {
         ++skipbs;
-        for (int j = l; j < n; j += 64) sol.st(i * n + j, NT<K, CX>::zero());
-        wsync();
+        for (int j = l; j < n; j += Team<TW>::N) sol.st(i * n + j, NT<K, CX>::zero());
+        Team<TW>::sync();
       } else {
         if (firstbs) {
           f.newtail = i;
           firstbs = false;
         }
-        any_qrbs<K, CX>(n, w, rhs, i * n, sol, i * n);
+        any_qrbs<K, CX, TW>(n, w, rhs, i * n, sol, i * n);
       }
     }
     f.up = skipup;
@@ -538,7 +560,7 @@ __device__ void qrbs_solve(int n, int degp1, int tailidx, const M &mat, const Ar
 
 // the supports of a row system (shared by every system of a batch)
 struct RowSys {
-  int dim, nmono, nvmax, nbrmax;
+  int dim, nmono, nvmax, nbrmax, nfacmax;  // nfacmax: most factors of a common factor
   const int *monoptr, *nvr, *idxptr, *idx;
   const int *exp;  // exponents parallel to idx, nullptr when all are 1
   // A system in the column representation (the column Newton method),
@@ -566,56 +588,89 @@ template <int K> __device__ __forceinline__ mdr<K> times_exp(const mdr<K> &v, do
   return mul_d(v, e);
 }
 
-// coefficient k of x*y: x_0 y_k, then += x_i y_{k-i} (CPU_dbl2_product,
-// Convolutions/dbl2_convolutions_host.cpp:7-26)
-template <int K, bool CX, class FX, class FY>
-__device__ __forceinline__ typename NT<K, CX>::V cprod(const FX &x, const FY &y, int k) {
-  typename NT<K, CX>::V acc = NT<K, CX>::mul(x(0), y(k));
-  for (int i = 1; i <= k; ++i) acc = NT<K, CX>::mac(acc, x(i), y(k - i));
-  return acc;
+// Two truncated products of series at once by the Dp lanes (lane k < Dw) of a
+// component of a slot: coefficient k of x1*y1, then coefficient Dw-1-k of x2*y2
+// (when two), Dw + 1 multiply-adds on every lane where one lane per coefficient
+// of one product leaves half of them idle.  x1, ...: the rows' offsets in the
+// planar array E; part: the component of a complex number this lane forms (0
+// the real, 1 the imaginary part).  Each coefficient x_0 y_k, then += x_i
+// y_{k-i}, in the order of CPU_dbl2_product and CPU_cmplx2_product
+// (Convolutions/dbl2_convolutions_host.cpp:7-88).
+template <int K, bool CX>
+__device__ __forceinline__ void cprod2(const Arr<K, CX> &E, int part, int x1, int y1, int x2, int y2, int Dw,
+                                       int k, bool two, typename RealT<K>::type &r1,
+                                       typename RealT<K>::type &r2) {
+  typedef typename RealT<K>::type T;
+  const int T1 = two ? Dw + 1 : k + 1;
+  const size_t im = (size_t)K * E.m;
+  T acc = R<K>::zero();
+  for (int it = 0; it < T1; ++it) {
+    const bool second = it > k, first = it == 0 || it == k + 1;
+    const int xo = second ? x2 + (it - k - 1) : x1 + it, yo = second ? y2 + (Dw - it) : y1 + (k - it);
+    if constexpr (CX) {
+      // re: xr yr - xi yi, im: xi yr + xr yi
+      const T xa = R<K>::load(E.b + (part ? im : 0), E.m, xo), xb = R<K>::load(E.b + (part ? 0 : im), E.m, xo);
+      const T p = mul(xa, R<K>::load(E.b, E.m, yo));
+      T q = mul(xb, R<K>::load(E.b + im, E.m, yo));
+      acc = choose(first, p, add(acc, p));
+      q = choose(part == 0, neg(q), q);
+      acc = add(q, acc);
+    } else {
+      const T p = mul(R<K>::load(E.b, E.m, xo), R<K>::load(E.b, E.m, yo));
+      acc = choose(first, p, add(acc, p));
+    }
+    if (it == k) r1 = acc;
+  }
+  r2 = acc;
 }
 
 // value and gradient series of every polynomial at X (working degree Dw-1):
 // out row (p*(dim+1)+j) = d p / d x_j, row (p*(dim+1)+dim) = p, as
 // CPU_dbl2_poly_evaldiff with CPU_dbl2_poly_speel and CPU_dbl2_speel
 // (Polynomials/dbl2_polynomials_host.cpp, Convolutions/dbl2_monomials_host.cpp:28-87).
-// Slot s (Dp lanes) evaluates polynomials s, s + nslot, ...; lane k of a slot
-// owns coefficient k.  cst/cff planes: cst + p*D, cff + m*D with plane strides.
-// A monomial's coefficient is staged in the slot's row CF; with exponents
-// it is first multiplied by the common factor prod_j x_j^(e_j - 1), one
-// factor at a time in the order of idx (the first loop of
-// CPU_dbl2_evaluate_monomials, Newton/dbl2_systems_host.cpp:18-45), and each
-// derivative contribution is multiplied by its exponent before it is added.
+// A slot (Dp lanes per component) evaluates polynomials s, s + nslot, ...; its
+// lane k of a component owns coefficients k and Dw-1-k of two products.
+// cst/cff planes: cst + p*D, cff + m*D with plane strides.  E: the variables X
+// at row offsets j*D, then the slots' work rows of length Dp: the coefficient
+// C, the forward chain F (nvmax - 1 rows) and the backward chain B (nvmax - 2).
+// A monomial's coefficient is staged in C; with exponents it is first
+// multiplied by the common factor prod_j x_j^(e_j - 1), one factor at a time
+// in the order of idx (the first loop of CPU_dbl2_evaluate_monomials,
+// Newton/dbl2_systems_host.cpp:18-45), and each derivative contribution is
+// multiplied by its exponent before it is added.  The chains advance together,
+// one cprod2 a level; contributions to one row of OUT are added in the
+// reference's order, the team in step (r1 before r2).
 // (complex: the products of CPU_cmplx2_poly_evaldiff; no exponents)
-template <int K, bool CX>
+template <int K, bool CX, int TW>
 __device__ void eval_system(const RowSys &S, int D, int Dw, int Dp, const double *cst,
                             size_t cstride, const double *cff, size_t fstride,
-                            const Arr<K, CX> &X, const Arr<K, CX> &OUT, const Arr<K, CX> &FW,
-                            const Arr<K, CX> &BW, const Arr<K, CX> &CR, const Arr<K, CX> &CF) {
-  typedef NT<K, CX> N;
-  typedef typename N::V T;
-  const int l = lane_id(), nslot = 64 / Dp, s = l / Dp, k = l % Dp;
-  const int dim = S.dim, D1 = dim + 1;
-  const int eo = s * S.nvmax * D;  // this slot's work rows
-  const int co = s * D;            // this slot's coefficient row
-  auto xin = [&](int var) { return [&X, var, D](int j) { return X.ld(var * D + j); }; };
-  auto fw = [&](int r) { return [&FW, eo, r, D](int j) { return FW.ld(eo + r * D + j); }; };
-  auto bw = [&](int r) { return [&BW, eo, r, D](int j) { return BW.ld(eo + r * D + j); }; };
-  auto cf = [&CF, co](int j) { return CF.ld(co + j); };
+                            const Arr<K, CX> &E, const Arr<K, CX> &OUT) {
+  typedef typename RealT<K>::type T;
+  typedef Team<TW> Tm;
+  const int G = (CX ? 2 : 1) * Dp, nslot = Tm::N / G, s = Tm::id() / G, part = Tm::id() % G / Dp,
+            k = Tm::id() % Dp;
+  const int dim = S.dim, D1 = dim + 1, k2 = Dw - 1 - k;
+  const int nv0 = S.nvmax > 0 ? S.nvmax : 1;
+  const int rows = 1 + (nv0 - 1) + (nv0 > 2 ? nv0 - 2 : 0);
+  const int C = dim * D + s * rows * Dp, F = C + Dp, B = F + (nv0 - 1) * Dp;
+  double *const Ep = E.b + (size_t)part * K * E.m, *const Op = OUT.b + (size_t)part * K * OUT.m;
+  auto keep = [&](int row, int q, const T &v) { R<K>::store(Ep, E.m, row + q, v); };
+  // levels of the products of a monomial of nv variables, see below
+  auto levels = [&](int nv) {
+    return nv < 2 ? nv : nv == 2 ? 2 + (S.column != 0) : nv + (nv - 2) / 2;
+  };
+  int nlev = levels(S.nvmax);
+  if (S.column && S.nvmax > 2 && nlev < 3) nlev = 3;
   for (int r0 = 0; r0 < dim; r0 += nslot) {
     const int p = r0 + s;
-    const bool on = (p < dim) && (k < Dw);
+    const bool on = s < nslot && p < dim && k < Dw;
     if (on) {
-      if constexpr (CX) {
-        OUT.st((p * D1 + dim) * D + k, N::ld(cst, cstride, (size_t)p * D + k));
-      } else {
-        // column systems (cst null): 0, or -1 in the last equation
-        T c0 = N::zero();
-        if (cst) c0 = N::ld(cst, cstride, (size_t)p * D + k);
-        else if (S.negone && p == dim - 1 && k == 0) c0 = N::neg(N::one());
-        OUT.st((p * D1 + dim) * D + k, c0);
-      }
-      for (int j = 0; j < dim; ++j) OUT.st((p * D1 + j) * D + k, N::zero());
+      // column systems (cst null): 0, or -1 in the last equation
+      T c0 = R<K>::zero();
+      if (cst) c0 = R<K>::load(cst + (size_t)part * K * cstride, cstride, (size_t)p * D + k);
+      else if (S.negone && p == dim - 1 && k == 0) c0 = R<K>::from(-1.0);
+      R<K>::store(Op, OUT.m, (p * D1 + dim) * D + k, c0);
+      for (int j = 0; j < dim; ++j) R<K>::store(Op, OUT.m, (p * D1 + j) * D + k, R<K>::zero());
     }
     const int nb = (p < dim) ? S.monoptr[p + 1] - S.monoptr[p] : 0;
     for (int mi = 0; mi < S.nbrmax; ++mi) {
@@ -624,91 +679,117 @@ __device__ void eval_system(const RowSys &S, int D, int Dw, int Dp, const double
       const int nv = act ? S.nvr[mono] : 0;
       const int *ix = S.idx + (act ? S.idxptr[mono] : 0);
       const int *ex = (!CX && act && S.exp) ? S.exp + S.idxptr[mono] : nullptr;
+      auto X = [&](int j) { return ix[j] * D; };
       // v times the exponent of variable position j (positions with
-      // exponent 1 are added as they are)
-      auto addto = [&](int row, const T &v, int j) {
-        const int o = (p * D1 + row) * D + k;
-        if constexpr (CX) {
-          OUT.st(o, N::add(OUT.ld(o), v));
-        } else {
-          const int e = (ex && j >= 0) ? ex[j] : 1;
-          const T ve = e > 1 ? times_exp(v, (double)e) : v;
-          OUT.st(o, S.assign ? ve : add(OUT.ld(o), ve));
-        }
+      // exponent 1 are added as they are) to coefficient q of an OUT row
+      auto addto = [&](int row, int q, const T &v, int j) {
+        const int o = (p * D1 + row) * D + q;
+        const int e = (ex && j >= 0) ? ex[j] : 1;
+        const T ve = e > 1 ? times_exp(v, (double)e) : v;
+        R<K>::store(Op, OUT.m, o, (!CX && S.assign) ? ve : add(R<K>::load(Op, OUT.m, o), ve));
       };
-      if constexpr (CX) {
-        if (act) CF.st(co + k, N::ld(cff, fstride, (size_t)mono * D + k));
-      } else if (act) {
+      if (act) {
         const size_t cm = S.cmap ? (size_t)S.cmap[mono] : (size_t)mono;
-        CF.st(co + k, cff ? N::ld(cff, fstride, cm * D + k) : (k == 0 ? N::one() : N::zero()));
+        T c = R<K>::from(k == 0 ? 1.0 : 0.0);
+        if (cff) c = R<K>::load(cff + (size_t)part * K * fstride, fstride, cm * D + k);
+        keep(C, k, c);
       }
-      wsync();
-      if (ex) {
-        for (int j = 0; j < nv; ++j)
-          for (int e = 1; e < ex[j]; ++e) {
-            const T a = cprod<K, CX>(xin(ix[j]), cf, k);
-            wsync();
-            CF.st(co + k, a);
-            wsync();
+      Tm::sync();
+      // the common factor, factor f of at most nfacmax: variable position fj
+      // while e of its e_j - 1 factors are taken
+      for (int f = 0, fj = 0, fe = 0; f < S.nfacmax; ++f) {
+        T a = R<K>::zero(), unused;
+        bool have = false;
+        if (ex) {
+          while (fj < nv && fe >= ex[fj] - 1) { ++fj; fe = 0; }
+          have = fj < nv;
+          if (have) {
+            cprod2<K, CX>(E, part, X(fj), C, 0, 0, Dw, k, false, a, unused);
+            ++fe;
           }
-      }
-      if (nv == 1) {
-        const T f = cprod<K, CX>(xin(ix[0]), cf, k);
-        addto(dim, f, -1);
-        addto(ix[0], cf(k), 0);
-      } else if (nv == 2) {
-        // the value: (c x_a) x_b in a polynomial, (x_a x_b) c in a column
-        // system (real only)
-        bool col = false;
-        if constexpr (!CX) col = S.column != 0;
-        const T f0 = cprod<K, CX>(cf, xin(ix[0]), k);
-        if (col) FW.st(eo + k, cprod<K, CX>(xin(ix[0]), xin(ix[1]), k));
-        else FW.st(eo + k, f0);
-        addto(ix[1], f0, 1);
-        const T b0 = cprod<K, CX>(cf, xin(ix[1]), k);
-        addto(ix[0], b0, 0);
-        wsync();
-        if (col) addto(dim, cprod<K, CX>(fw(0), cf, k), -1);
-        else addto(dim, cprod<K, CX>(fw(0), xin(ix[1]), k), -1);
-      } else if (nv > 2) {
-        // forward and backward chains advance together
-        FW.st(eo + k, cprod<K, CX>(cf, xin(ix[0]), k));
-        BW.st(eo + k, cprod<K, CX>(xin(ix[nv - 1]), xin(ix[nv - 2]), k));
-        wsync();
-        for (int j = 1; j < nv; ++j) {
-          FW.st(eo + j * D + k, cprod<K, CX>(fw(j - 1), xin(ix[j]), k));
-          if (j < nv - 2) BW.st(eo + j * D + k, cprod<K, CX>(bw(j - 1), xin(ix[nv - 2 - j]), k));
-          wsync();
         }
-        const T blast = cprod<K, CX>(bw(nv - 3), cf, k);
-        wsync();
-        BW.st(eo + (nv - 3) * D + k, blast);
-        wsync();
-        if (nv == 3) {
-          CR.st(eo + k, cprod<K, CX>(fw(0), xin(ix[2]), k));
-        } else {
-          for (int j = 0; j < nv - 3; ++j) CR.st(eo + j * D + k, cprod<K, CX>(fw(j), bw(nv - 4 - j), k));
-          CR.st(eo + (nv - 3) * D + k, cprod<K, CX>(fw(nv - 3), xin(ix[nv - 1]), k));
-        }
-        addto(dim, FW.ld(eo + (nv - 1) * D + k), -1);
-        addto(ix[nv - 1], FW.ld(eo + (nv - 2) * D + k), nv - 1);
-        addto(ix[0], BW.ld(eo + (nv - 3) * D + k), 0);
-        for (int j = 1; j < nv - 1; ++j) addto(ix[j], CR.ld(eo + (j - 1) * D + k), j);
+        Tm::sync();
+        if (have) keep(C, k, a);
+        Tm::sync();
       }
-      wsync();
+      if (nv == 1) addto(ix[0], k, R<K>::load(Ep, E.m, C + k), 0);
+      for (int t = 0; t < nlev; ++t) {
+        // two products x1 y1, x2 y2 (-1: none), the rows that keep them (-1:
+        // none), the OUT rows they are added to (-1: none) and the exponents'
+        // positions: for nv > 2 the chains f_t = f_{t-1} x_t (f_{-1} = c) and
+        // b_t = b_{t-1} x_{nv-2-t} (b_{-1} = x_{nv-1}) together, then c b_{nv-3}
+        // beside f_{nv-2}, then the value f_{nv-1} and the cross products f_j
+        // b_{nv-4-j} (the last f_{nv-3} x_{nv-1}) in order; for two variables
+        // the value is (c x_a) x_b in a polynomial, (x_a x_b) c in a column
+        // system
+        int x1 = -1, y1 = 0, x2 = -1, y2 = 0, d1 = -1, d2 = -1, o1 = -1, o2 = -1, e1 = -1, e2 = -1;
+        auto cross = [&](int j, int &x, int &y, int &o, int &e) {
+          x = F + j * Dp;
+          y = j < nv - 3 ? B + (nv - 4 - j) * Dp : X(nv - 1);
+          o = ix[j + 1];
+          e = j + 1;
+        };
+        if (nv == 1) {
+          if (t == 0) { x1 = X(0); y1 = C; o1 = dim; }
+        } else if (nv == 2) {
+          if (t == 0) {
+            x1 = C; y1 = X(0); o1 = ix[1]; e1 = 1;
+            if (!S.column) d1 = F;
+            x2 = C; y2 = X(1); o2 = ix[0]; e2 = 0;
+          } else if (!S.column) {
+            if (t == 1) { x1 = F; y1 = X(1); o1 = dim; }
+          } else if (t == 1) {
+            x1 = X(0); y1 = X(1); d1 = F;
+          } else if (t == 2) {
+            x1 = F; y1 = C; o1 = dim;
+          }
+        } else if (nv > 2) {
+          if (t <= nv - 3) {
+            x1 = t ? F + (t - 1) * Dp : C; y1 = X(t); d1 = F + t * Dp;
+            x2 = t ? B + (t - 1) * Dp : X(nv - 1); y2 = X(nv - 2 - t); d2 = B + t * Dp;
+          } else if (t == nv - 2) {
+            x1 = F + (t - 1) * Dp; y1 = X(t); d1 = F + t * Dp; o1 = ix[nv - 1]; e1 = nv - 1;
+            x2 = B + (t - 1) * Dp; y2 = C; o2 = ix[0]; e2 = 0;
+          } else if (t == nv - 1) {
+            x1 = F + (t - 1) * Dp; y1 = X(t); o1 = dim;
+            cross(0, x2, y2, o2, e2);
+          } else {
+            const int j = 2 * (t - nv) + 1;
+            if (j <= nv - 3) cross(j, x1, y1, o1, e1);
+            if (j + 1 <= nv - 3) cross(j + 1, x2, y2, o2, e2);
+          }
+        }
+        T r1, r2;
+        const bool have = act && x1 >= 0, two = have && x2 >= 0;
+        if (have) {
+          cprod2<K, CX>(E, part, x1, y1, x2, y2, Dw, k, two, r1, r2);
+          if (o1 >= 0) addto(o1, k, r1, e1);
+        }
+        Tm::sync();
+        if (have) {
+          if (two && o2 >= 0) addto(o2, k2, r2, e2);
+          if (d1 >= 0) keep(d1, k, r1);
+          if (two && d2 >= 0) keep(d2, k2, r2);
+        }
+        Tm::sync();
+      }
     }
   }
-  wsync();
+  Tm::sync();
 }
 
 // ------------------------------------------------------------ kernels
 
+// numbers of a system's LDS: X with the evaluation's work rows behind it (E)
+// and the solve's vectors and work arrays share it after X (SOLVE), the
+// Jacobian and value series (OUT; the right-hand side is formed in place of
+// the value rows), Q and R.
 struct NewtonLayout {
-  int X, OUT, RHS, SOL, Q, R, V, W1, W2, WRK, SC, FW, BW, CR, CF;  // sizes in numbers
+  int E, X, SOLVE, OUT, Q;
   // P doubles per number: K (real) or 2K (complex)
   __host__ __device__ size_t bytes(int P) const {
-    return sizeof(double) * (size_t)P *
-           ((size_t)X + OUT + RHS + SOL + Q + R + V + W1 + W2 + WRK + SC + FW + BW + CR + CF);
+    const int ev = E - X, tail = ev > SOLVE ? ev : SOLVE;
+    return sizeof(double) * (size_t)P * ((size_t)X + tail + OUT + 2 * (size_t)Q);
   }
 };
 
@@ -718,13 +799,27 @@ __host__ __device__ inline int pow2_at_least(int d) {
   return p;
 }
 
-__host__ __device__ inline NewtonLayout newton_layout(const RowSys &S, int D) {
-  const int n = S.dim, nslot = 64 / pow2_at_least(D), ev = nslot * (S.nvmax > 0 ? S.nvmax : 1) * D;
+__host__ __device__ inline NewtonLayout newton_layout(const RowSys &S, int D, int TW, bool CX) {
+  const int n = S.dim, nv = S.nvmax > 0 ? S.nvmax : 1, rows = 1 + (nv - 1) + (nv > 2 ? nv - 2 : 0);
   NewtonLayout L;
-  L.X = n * D; L.OUT = n * (n + 1) * D; L.RHS = D * n; L.SOL = D * n;
-  L.Q = n * n; L.R = n * n; L.V = n; L.W1 = n; L.W2 = n; L.WRK = n; L.SC = 3;
-  L.FW = ev; L.BW = ev; L.CR = ev; L.CF = nslot * D;
+  L.X = n * D;
+  // 64 TW lanes, one per coefficient (and component) of a slot's rows
+  L.E = L.X + 64 * TW / (CX ? 2 : 1) * rows;
+  L.SOLVE = D * n + 4 * n + 3;  // SOL, v, w1, w2, wrk, scalars
+  L.OUT = n * (n + 1) * D;
+  L.Q = n * n;
   return L;
+}
+
+// wavefronts of a team: one while the systems fill the chip; with fewer
+// systems than 2 per compute unit (or more lanes than a wavefront's needed for
+// one slot) as many as evaluate all polynomials at once, up to 4
+inline int team_waves(const RowSys &S, int D, bool CX, int nsys) {
+  const int G = (CX ? 2 : 1) * pow2_at_least(D);
+  int tw = G > 64 ? 2 : 1;
+  if (nsys <= 512)
+    while (tw < 4 && 64 * tw < S.dim * G) tw *= 2;
+  return tw;
 }
 
 template <int K, bool CX = false>
@@ -741,43 +836,57 @@ __device__ LinWork<K, CX> carve_lin(double *&p, int n) {
 // [nbsteps][K][nsys][dim][D]; Q, R [K][nsys][dim][dim].  Column systems:
 // cst null, cff null for unit coefficients, mb [K][nm][dim][D] (nm = nsys
 // or 1); rows: mb null.
-template <int K, bool CX>
-__global__ void __launch_bounds__(512)
+template <int K, bool CX, int TW>
+__global__ void __launch_bounds__(64 * TW)
 row_newton_kernel(RowSys S, int deg, int nbsteps, int nsys, const double *cst, int cshared,
                   const double *cff, int fshared, const double *mb, int mshared, double *x,
                   int *steps_out, int *wdeg_out, int *tail_out, int *up_out, int *bs_out,
                   double *hist, double *Qo, double *Ro) {
   typedef NT<K, CX> N;
+  typedef Team<TW> Tm;
   extern __shared__ double lds[];
-  const int D = deg + 1, n = S.dim, Dp = pow2_at_least(D);
-  const NewtonLayout L = newton_layout(S, D);
-  const int wave = threadIdx.x >> 6, l = lane_id();
-  const int sysid = blockIdx.x * (blockDim.x >> 6) + wave;
-  if (sysid >= nsys) return;
-  double *p = lds + (size_t)wave * (L.bytes(N::P) / sizeof(double));
-  const Arr<K, CX> X = carve<K, CX>(p, L.X), OUT = carve<K, CX>(p, L.OUT),
-                   RHS = carve<K, CX>(p, L.RHS), SOL = carve<K, CX>(p, L.SOL);
-  const LinWork<K, CX> w = carve_lin<K, CX>(p, n);
-  const Arr<K, CX> FW = carve<K, CX>(p, L.FW), BW = carve<K, CX>(p, L.BW),
-                   CR = carve<K, CX>(p, L.CR), CF = carve<K, CX>(p, L.CF);
+  const int D = deg + 1, n = S.dim, D1 = n + 1;
+  const NewtonLayout L = newton_layout(S, D, TW, CX);
+  const int l = Tm::id(), sysid = blockIdx.x;
+  double *p = lds;
+  const Arr<K, CX> OUT = carve<K, CX>(p, L.OUT);
+  LinWork<K, CX> w;
+  w.q = carve<K, CX>(p, L.Q);
+  w.r = carve<K, CX>(p, L.Q);
+  // E is planar over X and the work rows, whose place is the solve's arrays'
+  // between evaluations
+  const int tail = L.E - L.X > L.SOLVE ? L.E - L.X : L.SOLVE;
+  const Arr<K, CX> E{p, L.X + tail};
+  auto sub_arr = [&](int off) { return Arr<K, CX>{E.b + L.X + off, E.m}; };
+  const Arr<K, CX> SOL = sub_arr(0);
+  w.v = sub_arr(D * n); w.w1 = sub_arr(D * n + n); w.w2 = sub_arr(D * n + 2 * n);
+  w.wrk = sub_arr(D * n + 3 * n); w.sc = sub_arr(D * n + 4 * n);
+  // right-hand side k of equation i in place of the value's coefficient
+  struct Rhs {
+    Arr<K, CX> a;
+    int n, D;
+    __device__ int at(int t) const { return (t % n * (n + 1) + n) * D + t / n; }
+    __device__ typename N::V ld(int t) const { return a.ld(at(t)); }
+    __device__ void st(int t, const typename N::V &v) const { a.st(at(t), v); }
+  };
+  const Rhs RHS{OUT, n, D};
   const size_t xs = (size_t)nsys * n * D, xb = (size_t)sysid * n * D;
   const size_t cs = (size_t)(cshared ? 1 : nsys) * n * D;
   const size_t fs = (size_t)(fshared ? 1 : nsys) * S.ncff * D;
   const size_t ms = (size_t)(mshared ? 1 : nsys) * n * D, mo = mshared ? 0 : (size_t)sysid * n * D;
   const double *cbase = cst ? cst + (cshared ? 0 : (size_t)sysid * n * D) : nullptr;
   const double *fbase = cff ? cff + (fshared ? 0 : (size_t)sysid * S.ncff * D) : nullptr;
-  for (int t = l; t < n * D; t += 64) X.st(t, N::ld(x, xs, xb + t));
-  wsync();
-  const int D1 = n + 1;
+  for (int t = l; t < n * D; t += Tm::N) E.st(t, N::ld(x, xs, xb + t));
+  Tm::sync();
   auto jac = [&](int j, int r, int c) { return OUT.ld((r * D1 + c) * D + j); };
   Flags f{1, 0, 0, 0, 1};
   int tailidx = 1, wrkdeg = 0, stepcnt = 0;
   for (int step = 0; step < nbsteps; ++step) {
     const int Dw = wrkdeg + 1;
-    eval_system<K, CX>(S, D, Dw, Dp, cbase, cs, fbase, fs, X, OUT, FW, BW, CR, CF);
-    for (int t = l; t < Dw * n; t += 64) {
+    eval_system<K, CX, TW>(S, D, Dw, pow2_at_least(Dw), cbase, cs, fbase, fs, E, OUT);
+    for (int t = l; t < Dw * n; t += Tm::N) {
       const int kk = t / n, i = t % n;
-      const typename N::V fv = OUT.ld((i * D1 + n) * D + kk);
+      const typename N::V fv = RHS.ld(t);
       if constexpr (CX) {
         RHS.st(t, N::neg(fv));
       } else {
@@ -786,15 +895,16 @@ row_newton_kernel(RowSys S, int deg, int nbsteps, int nsys, const double *cst, i
       }
       SOL.st(t, N::zero());
     }
-    wsync();
+    Tm::sync();
     f.newtail = tailidx;
-    qrbs_solve<K, CX>(n, Dw, tailidx, jac, RHS, SOL, w, f);
+    qrbs_solve<K, CX, TW>(n, Dw, tailidx, jac, RHS, SOL, w, f);
     tailidx = f.newtail;
-    for (int t = l; t < n * Dw; t += 64) {
+    Tm::sync();
+    for (int t = l; t < n * Dw; t += Tm::N) {
       const int i = t / Dw, kk = t % Dw;
-      if (kk >= tailidx - 1) X.st(i * D + kk, N::add(X.ld(i * D + kk), SOL.ld(kk * n + i)));
+      if (kk >= tailidx - 1) E.st(i * D + kk, N::add(E.ld(i * D + kk), SOL.ld(kk * n + i)));
     }
-    wsync();
+    Tm::sync();
     if (l == 0) {
       const size_t o = (size_t)sysid * nbsteps + step;
       if (wdeg_out) wdeg_out[o] = wrkdeg;
@@ -804,16 +914,16 @@ row_newton_kernel(RowSys S, int deg, int nbsteps, int nsys, const double *cst, i
     }
     if (hist) {
       double *h = hist + (size_t)step * N::P * xs;
-      for (int t = l; t < n * D; t += 64) N::st(h, xs, xb + t, X.ld(t));
+      for (int t = l; t < n * D; t += Tm::N) N::st(h, xs, xb + t, E.ld(t));
     }
     ++stepcnt;
     if (tailidx >= deg) break;
     wrkdeg = wrkdeg + 1 + wrkdeg / 2;
     if (wrkdeg > deg) wrkdeg = deg;
   }
-  for (int t = l; t < n * D; t += 64) N::st(x, xs, xb + t, X.ld(t));
+  for (int t = l; t < n * D; t += Tm::N) N::st(x, xs, xb + t, E.ld(t));
   const size_t qs = (size_t)nsys * n * n, qb = (size_t)sysid * n * n;
-  for (int t = l; t < n * n; t += 64) {
+  for (int t = l; t < n * n; t += Tm::N) {
     if (Qo) N::st(Qo, qs, qb + t, w.q.ld(t));
     if (Ro) N::st(Ro, qs, qb + t, w.r.ld(t));
   }
@@ -833,7 +943,7 @@ houseqr_kernel(int n, int nb, const double *A, double *Qo, double *Ro) {
   double *p = lds + (size_t)wave * per;
   const LinWork<K, CX> w = carve_lin<K, CX>(p, n);
   const size_t s = (size_t)nb * n * n, o = (size_t)b * n * n;
-  any_houseqr<K, CX>(n, [&](int r, int c) { return N::ld(A, s, o + (size_t)r * n + c); }, w);
+  any_houseqr<K, CX, 1>(n, [&](int r, int c) { return N::ld(A, s, o + (size_t)r * n + c); }, w);
   for (int t = l; t < n * n; t += 64) {
     N::st(Qo, s, o + t, w.q.ld(t));
     N::st(Ro, s, o + t, w.r.ld(t));
@@ -870,7 +980,7 @@ qrbs_solve_kernel(int n, int degp1, int tailidx, int nb, const double *mat, doub
   wsync();
   Flags f{flags[b * 5], flags[b * 5 + 1], flags[b * 5 + 2], flags[b * 5 + 3], flags[b * 5 + 4]};
   auto m = [&](int j, int r, int c) { return N::ld(mat, ms, mo + ((size_t)j * n + r) * n + c); };
-  qrbs_solve<K, CX>(n, degp1, tailidx, m, RHS, SOL, w, f);
+  qrbs_solve<K, CX, 1>(n, degp1, tailidx, m, RHS, SOL, w, f);
   for (int t = l; t < degp1 * n; t += 64) {
     N::st(rhs, vs, vo + t, RHS.ld(t));
     N::st(sol, vs, vo + t, SOL.ld(t));
@@ -985,9 +1095,15 @@ int phc_rowsys_create_exp(phc_rowsys **out, int dim, const int *monoptr, const i
   }
   const int nidx = idxptr[nmono];
   bool any_exp = false;
+  int nfacmax = 0;
   for (int j = 0; exp && j < nidx; ++j) {
     PHC_REQUIRE(exp[j] >= 1 && exp[j] <= 64, "phc_rowsys_create: exponents must be in 1..64");
     any_exp = any_exp || exp[j] > 1;
+  }
+  for (int m = 0; exp && m < nmono; ++m) {
+    int nfac = 0;
+    for (int j = idxptr[m]; j < idxptr[m + 1]; ++j) nfac += exp[j] - 1;
+    if (nfac > nfacmax) nfacmax = nfac;
   }
   const size_t ints = (size_t)(dim + 1) + 2 * (size_t)nmono + 1 + nidx + (any_exp ? nidx : 0);
   phc_rowsys *s = new phc_rowsys();
@@ -1005,6 +1121,7 @@ int phc_rowsys_create_exp(phc_rowsys **out, int dim, const int *monoptr, const i
   if (any_exp) h.insert(h.end(), exp, exp + nidx);
   PHC_HIP(hipMemcpy(p, h.data(), sizeof(int) * h.size(), hipMemcpyHostToDevice));
   s->S.dim = dim; s->S.nmono = nmono; s->S.nvmax = nvmax; s->S.nbrmax = nbrmax;
+  s->S.nfacmax = nfacmax;
   s->S.monoptr = p; s->S.nvr = p + dim + 1; s->S.idxptr = p + dim + 1 + nmono;
   s->S.idx = p + dim + 1 + 2 * nmono + 1;
   s->S.exp = any_exp ? s->S.idx + nidx : nullptr;
@@ -1090,7 +1207,7 @@ int phc_rowsys_destroy(phc_rowsys *s) {
 int phc_rowsys_lds_bytes(const phc_rowsys *s, int K, int deg, size_t *bytes) {
   PHC_REQUIRE(s && bytes, "phc_rowsys_lds_bytes: null argument");
   PHC_REQUIRE(deg >= 0 && deg <= 63, "phc_rowsys_lds_bytes: deg must be in 0..63");
-  *bytes = newton_layout(s->S, deg + 1).bytes(K);
+  *bytes = newton_layout(s->S, deg + 1, 1, false).bytes(K);
   return 0;
 }
 
@@ -1124,23 +1241,32 @@ int row_newton(phc_rowsys *s, int K, int deg, int nbsteps, int nsys, const doubl
     PHC_REQUIRE(cst && cff && x, std::string(fn) + ": null coefficient or series array");
   }
   if (nsys == 0 || nbsteps == 0) return 0;
-  const size_t per = newton_layout(s->S, deg + 1).bytes(CX ? 2 * K : K);
+  const int P = CX ? 2 * K : K;
+  int tw = team_waves(s->S, deg + 1, CX, nsys);
+  // more wavefronts take more work rows
+  while (tw > 1 && newton_layout(s->S, deg + 1, tw, CX).bytes(P) > LDS_LIMIT && 32 * tw >= (CX ? 2 : 1) * pow2_at_least(deg + 1)) tw /= 2;
+  const size_t lds = newton_layout(s->S, deg + 1, tw, CX).bytes(P);
   int wv = 0;
-  if (waves_for(per, &wv) != 0) return -2;
-  const int grid = (nsys + wv - 1) / wv;
-  const size_t lds = per * wv;
+  if (waves_for(lds, &wv) != 0) return -2;
   hipStream_t st = (hipStream_t)stream;
+#define LAUNCH_TEAM(KK, TW)                                                                   \
+  do {                                                                                        \
+    PHC_HIP(hipFuncSetAttribute((const void *)row_newton_kernel<KK, CX, TW>,                 \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));       \
+    hipLaunchKernelGGL((row_newton_kernel<KK, CX, TW>), dim3(nsys), dim3(64 * TW), lds, st,   \
+                       s->S, deg, nbsteps, nsys, cst, cst_shared, cff, cff_shared, mb,        \
+                       mb_shared, x, steps, wdeg, tail, up, bs, history, Q, R);               \
+  } while (0)
 #define LAUNCH(KK)                                                                            \
   do {                                                                                        \
-    PHC_HIP(hipFuncSetAttribute((const void *)row_newton_kernel<KK, CX>,                     \
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));       \
-    hipLaunchKernelGGL((row_newton_kernel<KK, CX>), dim3(grid), dim3(64 * wv), lds, st, s->S, \
-                       deg, nbsteps, nsys, cst, cst_shared, cff, cff_shared, mb, mb_shared, \
-                       x, steps, wdeg, tail, up, bs, history, Q, R);                          \
+    if (tw == 1) LAUNCH_TEAM(KK, 1);                                                          \
+    else if (tw == 2) LAUNCH_TEAM(KK, 2);                                                     \
+    else LAUNCH_TEAM(KK, 4);                                                                  \
   } while (0)
   if (K == 1 && !CX) LAUNCH(1);
   else if (K == 2) LAUNCH(2);
   else LAUNCH(4);
+#undef LAUNCH_TEAM
 #undef LAUNCH
   PHC_HIP(hipGetLastError());
   return 0;
