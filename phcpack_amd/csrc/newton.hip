@@ -117,14 +117,21 @@ template <int K> struct NT<K, true> {
   __device__ static double mag(const V &a) { return fabs(R<K>::hi(a.re)) + fabs(R<K>::hi(a.im)); }
 };
 
-// a planar LDS (or global) array of m numbers with K limbs (2K planes when
-// complex)
+// an LDS array of numbers, the P limbs of each side by side (K, or 2K when
+// complex: a pair of limbs is one 16-byte access)
 template <int K, bool CX = false> struct Arr {
   typedef typename NT<K, CX>::V T;
+  static constexpr int P = NT<K, CX>::P;
   double *b;
-  int m;
-  __device__ T ld(int j) const { return NT<K, CX>::ld(b, m, j); }
-  __device__ void st(int j, const T &v) const { NT<K, CX>::st(b, m, j, v); }
+  __device__ T ld(int j) const { return NT<K, CX>::ld(b + j * P, 1, 0); }
+  __device__ void st(int j, const T &v) const { NT<K, CX>::st(b + j * P, 1, 0, v); }
+  // the real (part 0) or imaginary (1) part of number j
+  __device__ typename RealT<K>::type ldp(int j, int part) const {
+    return R<K>::load(b + j * P + part * K, 1, 0);
+  }
+  __device__ void stp(int j, int part, const typename RealT<K>::type &v) const {
+    R<K>::store(b + j * P + part * K, 1, 0, v);
+  }
 };
 
 __device__ __forceinline__ bool all_zero(double a) { return a == 0.0; }
@@ -146,9 +153,9 @@ template <int K> __device__ __forceinline__ mdr<K> choose(bool c, const mdr<K> &
   return r;
 }
 
-// carve a planar array of m numbers out of LDS
+// carve an array of m numbers out of LDS
 template <int K, bool CX = false> __device__ Arr<K, CX> carve(double *&p, int m) {
-  Arr<K, CX> a{p, m};
+  Arr<K, CX> a{p};
   p += (size_t)NT<K, CX>::P * m;
   return a;
 }
@@ -558,21 +565,28 @@ __device__ void qrbs_solve(int n, int degp1, int tailidx, const M &mat, const BV
 
 // ---------------------------------------------- polynomial system values
 
+// a monomial in one load: variable j in byte j of ix and its exponent in byte
+// j of ex (the first eight), the number of variables, its coefficient series
+struct MonoDesc {
+  unsigned long long ix, ex;
+  int nv, cm;
+};
+
 // the supports of a row system (shared by every system of a batch)
 struct RowSys {
   int dim, nmono, nvmax, nbrmax, nfacmax;  // nfacmax: most factors of a common factor
   const int *monoptr, *nvr, *idxptr, *idx;
+  const MonoDesc *desc;
   const int *exp;  // exponents parallel to idx, nullptr when all are 1
   // A system in the column representation (the column Newton method),
   // equation j holding monomial j of every column in column order: each
   // monomial is evaluated as CPU_dbl2_evaldiff does (a two-variable
   // monomial's value as (x_a x_b) c), the coefficient of row monomial m is
-  // coefficient series cmap[m] of the caller's ncff per system (unit series
+  // coefficient series desc[m].cm of the caller's ncff per system (unit series
   // when the coefficients are null: a monomial system), the constant is -1
   // in the last equation when negone and 0 elsewhere, and the right-hand
   // side of the linearized system is -(f - mb).
   int column, negone, ncff;
-  const int *cmap;
   // a monomial system (one monomial per equation): its value and
   // derivatives are stored, not added to zero, as
   // dbl2_linearize_evaldiff_output copies them (Newton/dbl2_systems_host.cpp:
@@ -592,7 +606,7 @@ template <int K> __device__ __forceinline__ mdr<K> times_exp(const mdr<K> &v, do
 // component of a slot: coefficient k of x1*y1, then coefficient Dw-1-k of x2*y2
 // (when two), Dw + 1 multiply-adds on every lane where one lane per coefficient
 // of one product leaves half of them idle.  x1, ...: the rows' offsets in the
-// planar array E; part: the component of a complex number this lane forms (0
+// array E; part: the component of a complex number this lane forms (0
 // the real, 1 the imaginary part).  Each coefficient x_0 y_k, then += x_i
 // y_{k-i}, in the order of CPU_dbl2_product and CPU_cmplx2_product
 // (Convolutions/dbl2_convolutions_host.cpp:7-88).
@@ -601,25 +615,29 @@ __device__ __forceinline__ void cprod2(const Arr<K, CX> &E, int part, int x1, in
                                        int k, bool two, typename RealT<K>::type &r1,
                                        typename RealT<K>::type &r2) {
   typedef typename RealT<K>::type T;
+  constexpr int P = Arr<K, CX>::P;
   const int T1 = two ? Dw + 1 : k + 1;
-  const size_t im = (size_t)K * E.m;
   T acc = R<K>::zero();
+  // offsets of the next x and y, in limbs
+  int xo = x1 * P, yo = (y1 + k) * P;
   for (int it = 0; it < T1; ++it) {
-    const bool second = it > k, first = it == 0 || it == k + 1;
-    const int xo = second ? x2 + (it - k - 1) : x1 + it, yo = second ? y2 + (Dw - it) : y1 + (k - it);
+    const T xr = R<K>::load(E.b + xo + (CX && part ? K : 0), 1, 0), yr = R<K>::load(E.b + yo, 1, 0);
+    const T p = mul(xr, yr);
+    acc = choose(it == 0 || it == k + 1, p, add(acc, p));
     if constexpr (CX) {
       // re: xr yr - xi yi, im: xi yr + xr yi
-      const T xa = R<K>::load(E.b + (part ? im : 0), E.m, xo), xb = R<K>::load(E.b + (part ? 0 : im), E.m, xo);
-      const T p = mul(xa, R<K>::load(E.b, E.m, yo));
-      T q = mul(xb, R<K>::load(E.b + im, E.m, yo));
-      acc = choose(first, p, add(acc, p));
+      const T xi = R<K>::load(E.b + xo + (part ? 0 : K), 1, 0), yi = R<K>::load(E.b + yo + K, 1, 0);
+      T q = mul(xi, yi);
       q = choose(part == 0, neg(q), q);
       acc = add(q, acc);
-    } else {
-      const T p = mul(R<K>::load(E.b, E.m, xo), R<K>::load(E.b, E.m, yo));
-      acc = choose(first, p, add(acc, p));
     }
-    if (it == k) r1 = acc;
+    xo += P;
+    yo -= P;
+    if (it == k) {
+      r1 = acc;
+      xo = x2 * P;
+      yo = (y2 + Dw - 1 - k) * P;
+    }
   }
   r2 = acc;
 }
@@ -653,8 +671,7 @@ __device__ void eval_system(const RowSys &S, int D, int Dw, int Dp, const double
   const int nv0 = S.nvmax > 0 ? S.nvmax : 1;
   const int rows = 1 + (nv0 - 1) + (nv0 > 2 ? nv0 - 2 : 0);
   const int C = dim * D + s * rows * Dp, F = C + Dp, B = F + (nv0 - 1) * Dp;
-  double *const Ep = E.b + (size_t)part * K * E.m, *const Op = OUT.b + (size_t)part * K * OUT.m;
-  auto keep = [&](int row, int q, const T &v) { R<K>::store(Ep, E.m, row + q, v); };
+  auto keep = [&](int row, int q, const T &v) { E.stp(row + q, part, v); };
   // levels of the products of a monomial of nv variables, see below
   auto levels = [&](int nv) {
     return nv < 2 ? nv : nv == 2 ? 2 + (S.column != 0) : nv + (nv - 2) / 2;
@@ -669,39 +686,48 @@ __device__ void eval_system(const RowSys &S, int D, int Dw, int Dp, const double
       T c0 = R<K>::zero();
       if (cst) c0 = R<K>::load(cst + (size_t)part * K * cstride, cstride, (size_t)p * D + k);
       else if (S.negone && p == dim - 1 && k == 0) c0 = R<K>::from(-1.0);
-      R<K>::store(Op, OUT.m, (p * D1 + dim) * D + k, c0);
-      for (int j = 0; j < dim; ++j) R<K>::store(Op, OUT.m, (p * D1 + j) * D + k, R<K>::zero());
+      OUT.stp((p * D1 + dim) * D + k, part, c0);
+      for (int j = 0; j < dim; ++j) OUT.stp((p * D1 + j) * D + k, part, R<K>::zero());
     }
-    const int nb = (p < dim) ? S.monoptr[p + 1] - S.monoptr[p] : 0;
+    const int m0 = on ? S.monoptr[p] : 0, nb = on ? S.monoptr[p + 1] - m0 : 0;
+    // the next monomial's description and coefficient are loaded while the
+    // current one is evaluated
+    MonoDesc next{0, 0, 0, 0};
+    T cnext = R<K>::zero();
+    auto fetch = [&](int mi) {
+      if (mi >= nb) return;
+      next = S.desc[m0 + mi];
+      cnext = R<K>::from(k == 0 ? 1.0 : 0.0);
+      if (cff) cnext = R<K>::load(cff + (size_t)part * K * fstride, fstride, (size_t)next.cm * D + k);
+    };
+    fetch(0);
     for (int mi = 0; mi < S.nbrmax; ++mi) {
-      const bool act = on && mi < nb;
-      const int mono = act ? S.monoptr[p] + mi : 0;
-      const int nv = act ? S.nvr[mono] : 0;
-      const int *ix = S.idx + (act ? S.idxptr[mono] : 0);
-      const int *ex = (!CX && act && S.exp) ? S.exp + S.idxptr[mono] : nullptr;
-      auto X = [&](int j) { return ix[j] * D; };
+      const bool act = mi < nb;
+      const MonoDesc md = next;
+      const T c = cnext;
+      fetch(mi + 1);
+      const int mono = m0 + mi, nv = act ? md.nv : 0;
+      const bool wide = nv > 8, powers = !CX && act && S.exp;
+      auto var = [&](int j) { return wide ? S.idx[S.idxptr[mono] + j] : (int)(md.ix >> (8 * j)) & 255; };
+      auto expo = [&](int j) { return wide ? S.exp[S.idxptr[mono] + j] : (int)(md.ex >> (8 * j)) & 255; };
+      auto X = [&](int j) { return var(j) * D; };
       // v times the exponent of variable position j (positions with
       // exponent 1 are added as they are) to coefficient q of an OUT row
       auto addto = [&](int row, int q, const T &v, int j) {
         const int o = (p * D1 + row) * D + q;
-        const int e = (ex && j >= 0) ? ex[j] : 1;
+        const int e = (powers && j >= 0) ? expo(j) : 1;
         const T ve = e > 1 ? times_exp(v, (double)e) : v;
-        R<K>::store(Op, OUT.m, o, (!CX && S.assign) ? ve : add(R<K>::load(Op, OUT.m, o), ve));
+        OUT.stp(o, part, (!CX && S.assign) ? ve : add(OUT.ldp(o, part), ve));
       };
-      if (act) {
-        const size_t cm = S.cmap ? (size_t)S.cmap[mono] : (size_t)mono;
-        T c = R<K>::from(k == 0 ? 1.0 : 0.0);
-        if (cff) c = R<K>::load(cff + (size_t)part * K * fstride, fstride, cm * D + k);
-        keep(C, k, c);
-      }
+      if (act) keep(C, k, c);
       Tm::sync();
       // the common factor, factor f of at most nfacmax: variable position fj
       // while e of its e_j - 1 factors are taken
       for (int f = 0, fj = 0, fe = 0; f < S.nfacmax; ++f) {
         T a = R<K>::zero(), unused;
         bool have = false;
-        if (ex) {
-          while (fj < nv && fe >= ex[fj] - 1) { ++fj; fe = 0; }
+        if (powers) {
+          while (fj < nv && fe >= expo(fj) - 1) { ++fj; fe = 0; }
           have = fj < nv;
           if (have) {
             cprod2<K, CX>(E, part, X(fj), C, 0, 0, Dw, k, false, a, unused);
@@ -712,7 +738,7 @@ __device__ void eval_system(const RowSys &S, int D, int Dw, int Dp, const double
         if (have) keep(C, k, a);
         Tm::sync();
       }
-      if (nv == 1) addto(ix[0], k, R<K>::load(Ep, E.m, C + k), 0);
+      if (nv == 1) addto(var(0), k, E.ldp(C + k, part), 0);
       for (int t = 0; t < nlev; ++t) {
         // two products x1 y1, x2 y2 (-1: none), the rows that keep them (-1:
         // none), the OUT rows they are added to (-1: none) and the exponents'
@@ -726,16 +752,16 @@ __device__ void eval_system(const RowSys &S, int D, int Dw, int Dp, const double
         auto cross = [&](int j, int &x, int &y, int &o, int &e) {
           x = F + j * Dp;
           y = j < nv - 3 ? B + (nv - 4 - j) * Dp : X(nv - 1);
-          o = ix[j + 1];
+          o = var(j + 1);
           e = j + 1;
         };
         if (nv == 1) {
           if (t == 0) { x1 = X(0); y1 = C; o1 = dim; }
         } else if (nv == 2) {
           if (t == 0) {
-            x1 = C; y1 = X(0); o1 = ix[1]; e1 = 1;
+            x1 = C; y1 = X(0); o1 = var(1); e1 = 1;
             if (!S.column) d1 = F;
-            x2 = C; y2 = X(1); o2 = ix[0]; e2 = 0;
+            x2 = C; y2 = X(1); o2 = var(0); e2 = 0;
           } else if (!S.column) {
             if (t == 1) { x1 = F; y1 = X(1); o1 = dim; }
           } else if (t == 1) {
@@ -748,8 +774,8 @@ __device__ void eval_system(const RowSys &S, int D, int Dw, int Dp, const double
             x1 = t ? F + (t - 1) * Dp : C; y1 = X(t); d1 = F + t * Dp;
             x2 = t ? B + (t - 1) * Dp : X(nv - 1); y2 = X(nv - 2 - t); d2 = B + t * Dp;
           } else if (t == nv - 2) {
-            x1 = F + (t - 1) * Dp; y1 = X(t); d1 = F + t * Dp; o1 = ix[nv - 1]; e1 = nv - 1;
-            x2 = B + (t - 1) * Dp; y2 = C; o2 = ix[0]; e2 = 0;
+            x1 = F + (t - 1) * Dp; y1 = X(t); d1 = F + t * Dp; o1 = var(nv - 1); e1 = nv - 1;
+            x2 = B + (t - 1) * Dp; y2 = C; o2 = var(0); e2 = 0;
           } else if (t == nv - 1) {
             x1 = F + (t - 1) * Dp; y1 = X(t); o1 = dim;
             cross(0, x2, y2, o2, e2);
@@ -844,7 +870,7 @@ row_newton_kernel(RowSys S, int deg, int nbsteps, int nsys, const double *cst, i
                   double *hist, double *Qo, double *Ro) {
   typedef NT<K, CX> N;
   typedef Team<TW> Tm;
-  extern __shared__ double lds[];
+  extern __shared__ __align__(16) double lds[];
   const int D = deg + 1, n = S.dim, D1 = n + 1;
   const NewtonLayout L = newton_layout(S, D, TW, CX);
   const int l = Tm::id(), sysid = blockIdx.x;
@@ -853,11 +879,10 @@ row_newton_kernel(RowSys S, int deg, int nbsteps, int nsys, const double *cst, i
   LinWork<K, CX> w;
   w.q = carve<K, CX>(p, L.Q);
   w.r = carve<K, CX>(p, L.Q);
-  // E is planar over X and the work rows, whose place is the solve's arrays'
+  // X and the evaluation's work rows, whose place is the solve's arrays'
   // between evaluations
-  const int tail = L.E - L.X > L.SOLVE ? L.E - L.X : L.SOLVE;
-  const Arr<K, CX> E{p, L.X + tail};
-  auto sub_arr = [&](int off) { return Arr<K, CX>{E.b + L.X + off, E.m}; };
+  const Arr<K, CX> E{p};
+  auto sub_arr = [&](int off) { return Arr<K, CX>{E.b + (L.X + off) * N::P}; };
   const Arr<K, CX> SOL = sub_arr(0);
   w.v = sub_arr(D * n); w.w1 = sub_arr(D * n + n); w.w2 = sub_arr(D * n + 2 * n);
   w.wrk = sub_arr(D * n + 3 * n); w.sc = sub_arr(D * n + 4 * n);
@@ -935,7 +960,7 @@ template <int K, bool CX>
 __global__ void __launch_bounds__(512)
 houseqr_kernel(int n, int nb, const double *A, double *Qo, double *Ro) {
   typedef NT<K, CX> N;
-  extern __shared__ double lds[];
+  extern __shared__ __align__(16) double lds[];
   const int wave = threadIdx.x >> 6, l = lane_id();
   const int b = blockIdx.x * (blockDim.x >> 6) + wave;
   if (b >= nb) return;
@@ -958,7 +983,7 @@ __global__ void __launch_bounds__(512)
 qrbs_solve_kernel(int n, int degp1, int tailidx, int nb, const double *mat, double *rhs,
                   double *sol, double *Qio, double *Rio, int *flags) {
   typedef NT<K, CX> N;
-  extern __shared__ double lds[];
+  extern __shared__ __align__(16) double lds[];
   const int wave = threadIdx.x >> 6, l = lane_id();
   const int b = blockIdx.x * (blockDim.x >> 6) + wave;
   if (b >= nb) return;
@@ -1059,9 +1084,29 @@ int waves_for(size_t per_wave, int *waves) {
 struct phc_rowsys {
   RowSys S;
   int *dmem;
-  int *cmem;   // column systems: the coefficient map
+  MonoDesc *ddesc;
   int nbrcol;  // column systems: the number of columns (0 for row systems)
 };
+
+namespace {
+// the monomials' descriptions (cmap: coefficient series of each, null: its own)
+int upload_desc(phc_rowsys *s, int nmono, const int *nvr, const int *idxptr, const int *idx,
+                const int *exp, const int *cmap) {
+  std::vector<MonoDesc> h(nmono > 0 ? nmono : 1, MonoDesc{0, 0, 0, 0});
+  for (int m = 0; m < nmono; ++m) {
+    h[m].nv = nvr[m];
+    h[m].cm = cmap ? cmap[m] : m;
+    for (int j = 0; j < nvr[m] && j < 8; ++j) {
+      h[m].ix |= (unsigned long long)idx[idxptr[m] + j] << (8 * j);
+      h[m].ex |= (unsigned long long)(exp ? exp[idxptr[m] + j] : 1) << (8 * j);
+    }
+  }
+  if (!s->ddesc) PHC_HIP(hipMalloc(&s->ddesc, sizeof(MonoDesc) * h.size()));
+  PHC_HIP(hipMemcpy(s->ddesc, h.data(), sizeof(MonoDesc) * h.size(), hipMemcpyHostToDevice));
+  s->S.desc = s->ddesc;
+  return 0;
+}
+}  // namespace
 
 extern "C" {
 
@@ -1126,6 +1171,10 @@ int phc_rowsys_create_exp(phc_rowsys **out, int dim, const int *monoptr, const i
   s->S.idx = p + dim + 1 + 2 * nmono + 1;
   s->S.exp = any_exp ? s->S.idx + nidx : nullptr;
   s->S.ncff = nmono;
+  if (upload_desc(s, nmono, nvr, idxptr, idx, exp, nullptr) != 0) {
+    phc_rowsys_destroy(s);
+    return -1;
+  }
   *out = s;
   return 0;
 }
@@ -1171,20 +1220,16 @@ int phc_colsys_create(phc_rowsys **out, int dim, int nbrcol, const int *nvr, con
   const int rc = phc_rowsys_create_exp(&s, dim, monoptr.data(), rnvr.data(), ridxptr.data(),
                                        ridx.data(), exps ? rexp.data() : nullptr);
   if (rc != 0) return rc;
-  int *dmap = nullptr;
-  if (!cmap.empty() && hipMalloc(&dmap, sizeof(int) * cmap.size()) != hipSuccess) {
-    phc_rowsys_destroy(s);
-    phc::set_error("phc_colsys_create: hipMalloc failed");
-    return -1;
-  }
-  if (dmap) PHC_HIP(hipMemcpy(dmap, cmap.data(), sizeof(int) * cmap.size(), hipMemcpyHostToDevice));
-  s->cmem = dmap;
   s->nbrcol = nbrcol;
   s->S.column = 1;
   s->S.negone = nbrcol > 1;
   s->S.assign = nbrcol == 1;
   s->S.ncff = ncff;
-  s->S.cmap = dmap;
+  if (upload_desc(s, (int)rnvr.size(), rnvr.data(), ridxptr.data(), ridx.data(),
+                  exps ? rexp.data() : nullptr, cmap.data()) != 0) {
+    phc_rowsys_destroy(s);
+    return -1;
+  }
   *out = s;
   return 0;
 }
@@ -1192,9 +1237,9 @@ int phc_colsys_create(phc_rowsys **out, int dim, int nbrcol, const int *nvr, con
 int phc_rowsys_destroy(phc_rowsys *s) {
   if (!s) return 0;
   hipError_t e = hipFree(s->dmem);
-  if (s->cmem) {
-    const hipError_t e2 = hipFree(s->cmem);
-    if (e == hipSuccess) e = e2;
+  if (s->ddesc) {
+    const hipError_t e1 = hipFree(s->ddesc);
+    if (e == hipSuccess) e = e1;
   }
   delete s;
   if (e != hipSuccess) {

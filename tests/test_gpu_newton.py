@@ -127,6 +127,32 @@ def test_row_newton_batch_matches_oracle(K, deg):
         assert np.array_equal(out["Q"][:, b], o["Q"]) and np.array_equal(out["R"][:, b], o["R"])
 
 
+@pytest.mark.parametrize("K,cx,dim,nper,nvar,deg,nsys", [(2, False, 10, 2, 9, 4, 3), (1, False, 3, 9, 2, 40, 2),
+                                                         (2, True, 2, 2, 2, 40, 2), (2, False, 2, 3, 1, 1, 600),
+                                                         (4, True, 5, 3, 4, 5, 600)])
+def test_row_newton_teams_match_oracle(K, cx, dim, nper, nvar, deg, nsys):
+    """monomials of more than eight variables, series longer than 32 (one slot
+    a wavefront, two wavefronts a slot in complex numbers), and more systems
+    than the several-wavefront teams take (one wavefront each)"""
+    from oraclelib import oracle_cx_row_newton, planted_cx_row_system
+    rng = np.random.default_rng(700 + dim + deg)
+    sup = random_supports(rng, dim, nper, nvar)
+    planted, solve = (planted_cx_row_system, oracle_cx_row_newton) if cx else (planted_row_system, oracle_row_newton)
+    systems = [planted(rng, K, dim, deg, supports=sup) for _ in range(3)]
+    pick = np.arange(nsys) % 3
+    cst = np.stack([systems[b][0].cst for b in pick], axis=1)
+    cff = np.stack([systems[b][0].cff for b in pick], axis=1)
+    x0 = np.stack([systems[b][2] for b in pick], axis=1)
+    out = _device_system(systems[0][0]).row_newton(K, deg, 6, cst, cff, x0, cplx=cx)
+    for b in sorted({0, min(1, nsys - 1), nsys - 1}):
+        o = solve(K, systems[pick[b]][0], systems[pick[b]][2], 6)
+        assert out["steps"][b] == o["steps"]
+        for k in ("wdeg", "tail", "up", "bs"):
+            assert np.array_equal(out[k][b, :o["steps"]], o[k]), (b, k)
+        # still bit for bit: a system whose Jacobian is singular ends in NaN in both
+        assert np.array_equal(out["x"][:, b], o["x"], equal_nan=True), b
+
+
 @pytest.mark.parametrize("K", (2,))
 def test_row_newton_shared_coefficients(K):
     """one system, many start series (shared coefficients)"""
