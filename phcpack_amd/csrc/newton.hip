@@ -180,8 +180,8 @@ __device__ double maxnorm(const A &v, int off, int n) {
 
 // ------------------------------------------------ Householder QR (square)
 
-// per-wave work arrays of the linear algebra; sc[0] = beta, sc[1] = v0
-// (complex: 1/v0), sc[2] = 1 when sigma = 0
+// per-wave work arrays of the linear algebra; sc[0] = beta, sc[1] = v0, sc[2]
+// = 1 when sigma = 0 (complex: sc[0] = beta and that flag, sc[1] = 1/v0)
 template <int K, bool CX = false> struct LinWork {
   Arr<K, CX> q, r, v, w1, w2, wrk, sc;
 };
@@ -295,18 +295,40 @@ __device__ void qrbs(int n, const LinWork<K> &w, const BV &bv, int bo, const Arr
   }
 }
 
+// The complex linear algebra works on components: two lanes form the real and
+// the imaginary part of a number, each with the operations of the reference's
+// host code in its order (a subtraction as the addition of the negated
+// number, which gives the same limbs).  One lane per number took twice as
+// long for each and the divisions of a row or a reflector one after another:
+// 1.0 M cycles for a 6 x 6 quad-double factorization, 170 k for a solve.
+
+// x - y or x + y
+template <class T> __device__ __forceinline__ T add_or_sub(const T &x, const T &y, bool minus) {
+  return add(x, choose(minus, neg(y), y));
+}
+
+// a value of lane src of the wavefront
+__device__ __forceinline__ double from_lane(double a, int src) { return __shfl(a, src, 64); }
+template <int K> __device__ __forceinline__ mdr<K> from_lane(const mdr<K> &a, int src) {
+  mdr<K> r;
+#pragma unroll
+  for (int i = 0; i < K; ++i) r.x[i] = __shfl(a.x[i], src, 64);
+  return r;
+}
+
 // Complex Q R = A (CPU_cmplx2_factors_houseqr with CPU_cmplx2_factors_house,
 // leftRupdate and rightQupdate, Matrices/dbl2_factorizations.cpp:441-533,
-// 567-627, 661-722, 766-822): lane 0 forms the Householder vector's scalars
-// (sigma = sum |x_i|^2, mu = sqrt(|x0|^2 + sigma) / |x0|, v0 = x0 - mu x0,
-// beta = 2 |v0|^2 / (sigma + |v0|^2), 1/v0 = conj(v0) / |v0|^2), the lanes
-// v_i = x_i / v0, then w1 = beta R^H v, w2 = beta Q v and the rank-one
-// updates R -= v w1^H, Q -= w2 v^H, every entry in the reference's order.
+// 567-627, 661-722, 766-822): the first wavefront forms the Householder
+// vector's scalars (sigma = sum |x_i|^2, mu = sqrt(|x0|^2 + sigma) / |x0|, v0 =
+// x0 - mu x0, beta = 2 |v0|^2 / (sigma + |v0|^2), 1/v0 = conj(v0) / |v0|^2),
+// both roots in one call and the last three quotients in another, then the
+// team v_i = x_i / v0, w1 = beta R^H v, w2 = beta Q v and the rank-one updates
+// R -= v w1^H, Q -= w2 v^H, every entry in the reference's order.
 template <int K, int TW, class A> __device__ void cx_houseqr(int n, const A &a, const LinWork<K, true> &w) {
   typedef typename RealT<K>::type T;
   typedef cplx<K> Z;
-  const int l = Team<TW>::id();
-  for (int t = l; t < n * n; t += Team<TW>::N) {
+  const int l = Team<TW>::id(), N = Team<TW>::N;
+  for (int t = l; t < n * n; t += N) {
     const int i = t / n, j = t % n;
     w.q.st(t, C<K>::from(i == j ? 1.0 : 0.0, 0.0));
     w.r.st(t, a(i, j));
@@ -314,180 +336,148 @@ template <int K, int TW, class A> __device__ void cx_houseqr(int n, const A &a, 
   Team<TW>::sync();
   for (int k = 0; k < n; ++k) {
     const int m = n - k;
-    if (l == 0) {
+    // the squares of the column's parts (w2 is free here)
+    for (int t = l; t < 2 * m; t += N) w.w2.stp(t >> 1, t & 1, sqr(w.r.ldp((k + (t >> 1)) * n + k, t & 1)));
+    Team<TW>::sync();
+    if (l < 64) {
       T sigma = R<K>::zero();
       for (int i = 1; i < m; ++i) {
-        const Z x = w.r.ld((k + i) * n + k);
-        sigma = add(sigma, sqr(x.re));
-        sigma = add(sigma, sqr(x.im));
+        sigma = add(sigma, w.w2.ldp(i, 0));
+        sigma = add(sigma, w.w2.ldp(i, 1));
       }
-      const bool zero = all_zero(sigma);
-      Z b;
-      b.re = R<K>::zero();
-      b.im = R<K>::from(zero ? 1.0 : 0.0);
-      w.sc.st(2, b);
-      if (zero) {
-        w.sc.st(0, C<K>::zero());
-        w.sc.st(1, C<K>::from(1.0, 0.0));
-      } else {
-        const Z x0 = w.r.ld(k * n + k);
-        T sqrx0 = add(sqr(x0.re), sqr(x0.im));
-        const T x0rad = R<K>::sqrt(sqrx0);
-        sqrx0 = add(sqrx0, sigma);
-        T mu = R<K>::sqrt(sqrx0);
-        Z v0;
+      const bool zero = all_zero(sigma), odd = l & 1;
+      T beta = R<K>::zero();
+      Z inv = C<K>::from(1.0, 0.0);
+      if (!zero) {
+        const T xc = w.r.ldp(k * n + k, odd);
+        const T sqrx0 = add(w.w2.ldp(0, 0), w.w2.ldp(0, 1));
+        // even lanes: sqrt(|x0|^2 + sigma), odd lanes: |x0|
+        const T rt = R<K>::sqrt(choose(odd, sqrx0, add(sqrx0, sigma)));
+        T mu = from_lane(rt, 0);
+        const T x0rad = from_lane(rt, 1);
+        // even lanes: v0.re, odd lanes: v0.im
+        T vc;
         if (all_zero(x0rad)) {
-          v0.re = neg(mu);
-          v0.im = R<K>::zero();
+          vc = choose(odd, R<K>::zero(), neg(mu));
         } else {
           mu = div(mu, x0rad);
-          v0.re = sub(x0.re, mul(mu, x0.re));
-          v0.im = sub(x0.im, mul(mu, x0.im));
+          vc = sub(xc, mul(mu, xc));
         }
-        const T sqrv0 = add(sqr(v0.re), sqr(v0.im));
+        const T v2 = sqr(vc);
+        const T sqrv0 = add(from_lane(v2, 0), from_lane(v2, 1));
         sigma = add(sigma, sqrv0);
-        T beta = div(sqrv0, sigma);
-        beta = mul_d(beta, 2.0);
-        Z inv;
-        inv.re = div(v0.re, sqrv0);
-        inv.im = neg(div(v0.im, sqrv0));
-        Z bz;
-        bz.re = beta;
-        bz.im = R<K>::zero();
-        w.sc.st(0, bz);
+        // lanes 0, 1: v0 / |v0|^2, lane 2: beta / 2
+        const T qt = div(choose(l == 2, sqrv0, vc), choose(l == 2, sigma, sqrv0));
+        beta = mul_d(from_lane(qt, 2), 2.0);
+        inv.re = from_lane(qt, 0);
+        inv.im = neg(from_lane(qt, 1));
+      }
+      if (l == 0) {
+        Z z;
+        z.re = beta;
+        z.im = R<K>::from(zero ? 1.0 : 0.0);
+        w.sc.st(0, z);
         w.sc.st(1, inv);
       }
     }
     Team<TW>::sync();
+    const T beta = w.sc.ldp(0, 0);
     {
       const Z inv = w.sc.ld(1);
-      const bool szero = R<K>::hi(w.sc.ld(2).im) != 0.0;
-      for (int i = l; i < m; i += Team<TW>::N) {
+      const bool szero = R<K>::hi(w.sc.ldp(0, 1)) != 0.0;
+      for (int t = l; t < 2 * m; t += N) {
+        const int i = t >> 1, part = t & 1;
         if (i == 0) {
-          w.v.st(0, C<K>::from(1.0, 0.0));
+          w.v.stp(0, part, R<K>::from(part ? 0.0 : 1.0));
         } else {
           const Z x = w.r.ld((k + i) * n + k);
-          if (szero) {
-            w.v.st(i, x);
-          } else {
-            Z v;
-            v.re = mul(x.re, inv.re);
-            v.re = sub(v.re, mul(x.im, inv.im));
-            v.im = mul(x.im, inv.re);
-            v.im = add(v.im, mul(x.re, inv.im));
-            w.v.st(i, v);
-          }
+          T v = part ? x.im : x.re;
+          if (!szero) v = add_or_sub(mul(v, inv.re), mul(part ? x.re : x.im, inv.im), part == 0);
+          w.v.stp(i, part, v);
         }
       }
     }
     Team<TW>::sync();
-    const T beta = w.sc.ld(0).re;
-    // w1[j-k] = beta * sum_i conj(R[i][j]) v[i-k]
-    for (int j = k + l; j < n; j += Team<TW>::N) {
-      Z s = C<K>::zero();
-      for (int i = k; i < n; ++i) {
-        const Z r = w.r.ld(i * n + j), v = w.v.ld(i - k);
-        T zre = mul(r.re, v.re);
-        zre = add(zre, mul(r.im, v.im));
-        T zim = mul(r.re, v.im);
-        zim = sub(zim, mul(r.im, v.re));
-        s.re = add(s.re, zre);
-        s.im = add(s.im, zim);
+    // w1[j-k] = beta * sum_i conj(R[i][j]) v[i-k], w2[i] = beta * sum_{j>=k}
+    // Q[i][j] v[j-k]
+    for (int t = l; t < 2 * (m + n); t += N) {
+      const bool one = t < 2 * m;
+      const int e = one ? t >> 1 : (t - 2 * m) >> 1, part = t & 1;
+      T s = R<K>::zero();
+      for (int q = 0; q < m; ++q) {
+        const Z x = one ? w.r.ld((k + q) * n + k + e) : w.q.ld(e * n + k + q), v = w.v.ld(q);
+        // w1: x.re v.re + x.im v.im, x.re v.im - x.im v.re
+        // w2: x.re v.re - x.im v.im, x.im v.re + x.re v.im
+        const bool im = part == 1, swap = !one && im;
+        const T p1 = mul(swap ? x.im : x.re, (im && one) ? v.im : v.re);
+        const T p2 = mul(swap ? x.re : x.im, (im && one) ? v.re : v.im);
+        s = add(s, add_or_sub(p1, p2, one == im));
       }
-      s.re = mul(beta, s.re);
-      s.im = mul(beta, s.im);
-      w.w1.st(j - k, s);
-    }
-    // w2[i] = beta * sum_{j>=k} Q[i][j] v[j-k]
-    for (int i = l; i < n; i += Team<TW>::N) {
-      Z s = C<K>::zero();
-      for (int j = k; j < n; ++j) {
-        const Z q = w.q.ld(i * n + j), v = w.v.ld(j - k);
-        T zre = mul(q.re, v.re);
-        zre = sub(zre, mul(q.im, v.im));
-        T zim = mul(q.im, v.re);
-        zim = add(zim, mul(q.re, v.im));
-        s.re = add(s.re, zre);
-        s.im = add(s.im, zim);
-      }
-      s.re = mul(beta, s.re);
-      s.im = mul(beta, s.im);
-      w.w2.st(i, s);
+      s = mul(beta, s);
+      if (one) w.w1.stp(e, part, s);
+      else w.w2.stp(e, part, s);
     }
     Team<TW>::sync();
     // R[i][j] -= v[i-k] conj(w1[j-k]);  Q[i][j] -= w2[i] conj(v[j-k])
-    for (int t = l; t < m * m; t += Team<TW>::N) {
-      const int i = k + t / m, j = k + t % m;
-      const Z v = w.v.ld(i - k), x = w.w1.ld(j - k);
-      Z r = w.r.ld(i * n + j);
-      T zre = mul(v.re, x.re);
-      zre = add(zre, mul(v.im, x.im));
-      T zim = mul(v.im, x.re);
-      zim = sub(zim, mul(v.re, x.im));
-      r.re = sub(r.re, zre);
-      r.im = sub(r.im, zim);
-      w.r.st(i * n + j, r);
-    }
-    for (int t = l; t < n * m; t += Team<TW>::N) {
-      const int i = t / m, j = k + t % m;
-      const Z x = w.w2.ld(i), v = w.v.ld(j - k);
-      Z q = w.q.ld(i * n + j);
-      T zre = mul(x.re, v.re);
-      zre = add(zre, mul(x.im, v.im));
-      T zim = mul(x.im, v.re);
-      zim = sub(zim, mul(x.re, v.im));
-      q.re = sub(q.re, zre);
-      q.im = sub(q.im, zim);
-      w.q.st(i * n + j, q);
+    for (int t = l; t < 2 * (m + n) * m; t += N) {
+      const int e = t >> 1, part = t & 1;
+      const bool one = e < m * m;
+      const int i = one ? e / m : (e - m * m) / m, j = one ? e % m : (e - m * m) % m;
+      const Z x = one ? w.v.ld(i) : w.w2.ld(i), y = one ? w.w1.ld(j) : w.v.ld(j);
+      const T z = add_or_sub(mul(part ? x.im : x.re, y.re), mul(part ? x.re : x.im, y.im), part == 1);
+      const Arr<K, true> &M = one ? w.r : w.q;
+      const int o = (one ? k + i : i) * n + k + j;
+      M.stp(o, part, sub(M.ldp(o, part), z));
     }
     Team<TW>::sync();
   }
 }
 
 // x = R^{-1} Q^H b (CPU_cmplx2_factors_qrbs and _backward, Matrices/
-// dbl2_factorizations.cpp:842-879, 142-200): b = bv[bo..], x = xv[xo..]
+// dbl2_factorizations.cpp:842-879, 142-200): b = bv[bo..], x = xv[xo..]; the
+// reciprocals of R's diagonal, which the reference forms row by row, first
 template <int K, int TW, class BV>
 __device__ void cx_qrbs(int n, const LinWork<K, true> &w, const BV &bv, int bo,
                         const Arr<K, true> &xv, int xo) {
   typedef typename RealT<K>::type T;
   typedef cplx<K> Z;
-  const int l = Team<TW>::id();
-  for (int i = l; i < n; i += Team<TW>::N) {
-    Z s = C<K>::zero();
+  const int l = Team<TW>::id(), N = Team<TW>::N;
+  for (int t = l; t < 2 * n; t += N) {
+    const int i = t >> 1, part = t & 1;
+    const Z u = w.r.ld(i * n + i);
+    const T den = add(mul(u.re, u.re), mul(u.im, u.im));
+    const T rc = div(part ? u.im : u.re, den);
+    w.w1.stp(i, part, choose(part == 1, neg(rc), rc));
+    T s = R<K>::zero();
     for (int j = 0; j < n; ++j) {
+      // re: + q.re b.re + q.im b.im, im: + q.re b.im - q.im b.re
       const Z q = w.q.ld(j * n + i), b = bv.ld(bo + j);
-      s.re = add(s.re, mul(q.re, b.re));
-      s.re = add(s.re, mul(q.im, b.im));
-      s.im = add(s.im, mul(q.re, b.im));
-      s.im = sub(s.im, mul(q.im, b.re));
+      s = add(s, mul(q.re, part ? b.im : b.re));
+      s = add_or_sub(s, mul(q.im, part ? b.re : b.im), part == 1);
     }
-    w.wrk.st(i, s);
+    w.wrk.stp(i, part, s);
   }
   Team<TW>::sync();
-  for (int i = l; i < n; i += Team<TW>::N) xv.st(xo + i, w.wrk.ld(i));
+  for (int i = l; i < n; i += N) xv.st(xo + i, w.wrk.ld(i));
   Team<TW>::sync();
   for (int j = n - 1; j >= 0; --j) {
-    if (l == j) {
-      const Z u = w.r.ld(j * n + j), x = xv.ld(xo + j);
-      const T den = add(mul(u.re, u.re), mul(u.im, u.im));
-      const T a1re = div(u.re, den), a1im = neg(div(u.im, den));
-      Z y;
-      y.re = sub(mul(x.re, a1re), mul(x.im, a1im));
-      y.im = add(mul(x.im, a1re), mul(x.re, a1im));
-      xv.st(xo + j, y);
+    T y;
+    if (l < 2) {
+      const Z x = xv.ld(xo + j), u = w.w1.ld(j);
+      y = add_or_sub(mul(l ? x.im : x.re, u.re), mul(l ? x.re : x.im, u.im), l == 0);
     }
     Team<TW>::sync();
+    if (l < 2) xv.stp(xo + j, l, y);
+    Team<TW>::sync();
     const Z xj = xv.ld(xo + j);
-    for (int i = l; i < j; i += Team<TW>::N) {
+    for (int t = l; t < 2 * j; t += N) {
+      // re: - u.re x.re + u.im x.im, im: - u.im x.re - u.re x.im
+      const int i = t >> 1, part = t & 1;
       const Z u = w.r.ld(i * n + j);
-      Z y = xv.ld(xo + i);
-      const T a1re = mul(u.re, xj.re), a1im = mul(u.im, xj.im);
-      const T a2re = mul(u.im, xj.re), a2im = mul(u.re, xj.im);
-      y.re = sub(y.re, a1re);
-      y.re = add(y.re, a1im);
-      y.im = sub(y.im, a2re);
-      y.im = sub(y.im, a2im);
-      xv.st(xo + i, y);
+      T v = xv.ldp(xo + i, part);
+      v = sub(v, mul(part ? u.im : u.re, xj.re));
+      v = add_or_sub(v, mul(part ? u.re : u.im, xj.im), part == 1);
+      xv.stp(xo + i, part, v);
     }
     Team<TW>::sync();
   }
@@ -537,11 +527,22 @@ __device__ void qrbs_solve(int n, int degp1, int tailidx, const M &mat, const BV
         ++skipup;
       } else {
         const int npair = (degp1 - i) * n;
-        for (int t = l; t < npair; t += Team<TW>::N) {
-          const int j = i + t / n, k = t % n;
-          T b = rhs.ld(j * n + k);
-          for (int L = 0; L < n; ++L) b = NT<K, CX>::msub(b, mat(j - i + 1, k, L), sol.ld((i - 1) * n + L));
-          rhs.st(j * n + k, b);
+        // a component of an entry per lane
+        constexpr int NC = CX ? 2 : 1;
+        for (int t = l; t < NC * npair; t += Team<TW>::N) {
+          const int e = t / NC, part = t % NC, j = i + e / n, k = e % n;
+          typename RealT<K>::type b = rhs.ldp(j * n + k, part);
+          for (int L = 0; L < n; ++L) {
+            const T a = mat(j - i + 1, k, L), x = sol.ld((i - 1) * n + L);
+            if constexpr (CX) {
+              // as NT::msub: re -= a.re x.re, += a.im x.im; im -= a.re x.im, -= a.im x.re
+              b = md::sub(b, md::mul(a.re, part ? x.im : x.re));
+              b = add_or_sub(b, md::mul(a.im, part ? x.re : x.im), part == 1);
+            } else {
+              b = md::sub(b, md::mul(a, x));
+            }
+          }
+          rhs.stp(j * n + k, part, b);
         }
       }
       Team<TW>::sync();
@@ -893,6 +894,8 @@ row_newton_kernel(RowSys S, int deg, int nbsteps, int nsys, const double *cst, i
     __device__ int at(int t) const { return (t % n * (n + 1) + n) * D + t / n; }
     __device__ typename N::V ld(int t) const { return a.ld(at(t)); }
     __device__ void st(int t, const typename N::V &v) const { a.st(at(t), v); }
+    __device__ typename RealT<K>::type ldp(int t, int part) const { return a.ldp(at(t), part); }
+    __device__ void stp(int t, int part, const typename RealT<K>::type &v) const { a.stp(at(t), part, v); }
   };
   const Rhs RHS{OUT, n, D};
   const size_t xs = (size_t)nsys * n * D, xb = (size_t)sysid * n * D;
