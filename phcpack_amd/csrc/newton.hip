@@ -604,42 +604,47 @@ template <int K> __device__ __forceinline__ mdr<K> times_exp(const mdr<K> &v, do
 }
 
 // Two truncated products of series at once by the Dp lanes (lane k < Dw) of a
-// component of a slot: coefficient k of x1*y1, then coefficient Dw-1-k of x2*y2
-// (when two), Dw + 1 multiply-adds on every lane where one lane per coefficient
-// of one product leaves half of them idle.  x1, ...: the rows' offsets in the
+// component of a slot: coefficient k of x1*y1, then coefficient Dw-1-k of x2*y2,
+// Dw + 1 multiply-adds on every lane where one lane per coefficient
+// of one product leaves half of them idle (no second product: x2 = y2 = 0).  x1, ...: the rows' offsets in the
 // array E; part: the component of a complex number this lane forms (0
 // the real, 1 the imaginary part).  Each coefficient x_0 y_k, then += x_i
 // y_{k-i}, in the order of CPU_dbl2_product and CPU_cmplx2_product
 // (Convolutions/dbl2_convolutions_host.cpp:7-88).
 template <int K, bool CX>
 __device__ __forceinline__ void cprod2(const Arr<K, CX> &E, int part, int x1, int y1, int x2, int y2, int Dw,
-                                       int k, bool two, typename RealT<K>::type &r1,
+                                       int k, typename RealT<K>::type &r1,
                                        typename RealT<K>::type &r2) {
   typedef typename RealT<K>::type T;
+  // Issue of instructions bounds it (reading ahead made it slower), so the
+  // trip count is uniform (without a second product the lanes go on with
+  // numbers that nobody reads), the turn to the second product is selects on
+  // one comparison, and up to double-double a sum starts from zero, to which
+  // the first product is added without a rounding: 60 -> 49 instructions a
+  // double-double multiply-add.
   constexpr int P = Arr<K, CX>::P;
-  const int T1 = two ? Dw + 1 : k + 1;
-  T acc = R<K>::zero();
-  // offsets of the next x and y, in limbs
-  int xo = x1 * P, yo = (y1 + k) * P;
-  for (int it = 0; it < T1; ++it) {
-    const T xr = R<K>::load(E.b + xo + (CX && part ? K : 0), 1, 0), yr = R<K>::load(E.b + yo, 1, 0);
-    const T p = mul(xr, yr);
-    acc = choose(it == 0 || it == k + 1, p, add(acc, p));
+  const double *px = E.b + x1 * P, *py = E.b + (y1 + k) * P, *const px2 = E.b + x2 * P,
+               *const py2 = E.b + (y2 + Dw - 1 - k) * P;
+  T acc = R<K>::zero(), first_sum = R<K>::zero();
+  bool first = true;
+#pragma unroll 2
+  for (int it = 0; it <= Dw; ++it) {
+    const T p = mul(R<K>::load(px + (CX && part ? K : 0), 1, 0), R<K>::load(py, 1, 0));
+    acc = K <= 2 ? add(acc, p) : choose(first, p, add(acc, p));
     if constexpr (CX) {
       // re: xr yr - xi yi, im: xi yr + xr yi
-      const T xi = R<K>::load(E.b + xo + (part ? 0 : K), 1, 0), yi = R<K>::load(E.b + yo + K, 1, 0);
-      T q = mul(xi, yi);
+      T q = mul(R<K>::load(px + (part ? 0 : K), 1, 0), R<K>::load(py + K, 1, 0));
       q = choose(part == 0, neg(q), q);
       acc = add(q, acc);
     }
-    xo += P;
-    yo -= P;
-    if (it == k) {
-      r1 = acc;
-      xo = x2 * P;
-      yo = (y2 + Dw - 1 - k) * P;
-    }
+    const bool turn = it == k;
+    first_sum = choose(turn, acc, first_sum);
+    if constexpr (K <= 2) acc = choose(turn, R<K>::zero(), acc);
+    first = turn;
+    px = turn ? px2 : px + P;
+    py = turn ? py2 : py - P;
   }
+  r1 = first_sum;
   r2 = acc;
 }
 
@@ -731,7 +736,7 @@ __device__ void eval_system(const RowSys &S, int D, int Dw, int Dp, const double
           while (fj < nv && fe >= expo(fj) - 1) { ++fj; fe = 0; }
           have = fj < nv;
           if (have) {
-            cprod2<K, CX>(E, part, X(fj), C, 0, 0, Dw, k, false, a, unused);
+            cprod2<K, CX>(E, part, X(fj), C, 0, 0, Dw, k, a, unused);
             ++fe;
           }
         }
@@ -789,7 +794,7 @@ __device__ void eval_system(const RowSys &S, int D, int Dw, int Dp, const double
         T r1, r2;
         const bool have = act && x1 >= 0, two = have && x2 >= 0;
         if (have) {
-          cprod2<K, CX>(E, part, x1, y1, x2, y2, Dw, k, two, r1, r2);
+          cprod2<K, CX>(E, part, x1, y1, two ? x2 : 0, two ? y2 : 0, Dw, k, r1, r2);
           if (o1 >= 0) addto(o1, k, r1, e1);
         }
         Tm::sync();
