@@ -269,9 +269,17 @@ template <int K> __device__ __forceinline__ cplx<K> group_sum(cplx<K> v, int G) 
   return v;
 }
 
-__device__ __forceinline__ double wave_max(double v) { return wave::max64(v); }
+// A value that every lane holds, from lane 0 in scalar registers: what follows
+// from it (the counters, the step control) is then scalar to the compiler as
+// well, branches need no lane masks, and it leaves the vector registers, of
+// which the variant with twelve wavefronts has too few.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ double uniform(double v) {
+  return __hiloint2double(uniform(__double2hiint(v)), uniform(__double2loint(v)));
+}
 
-__device__ __forceinline__ double wave_min(double v) { return wave::min64(v); }
+__device__ __forceinline__ double wave_max(double v) { return uniform(wave::max64(v)); }
+
 
 using wave::argmax_stage;
 
@@ -401,20 +409,25 @@ template <int K> __device__ void jacobian(const LProg &__restrict__ P, Path<K> &
   for (int e = l; e < P.n * P.n; e += 64) {
     // term t of the entry goes to accumulator (t - first) mod 4
     cplx<K> a[4] = {Cx::zero(), Cx::zero(), Cx::zero(), Cx::zero()};
-    const int t0 = P.jent[e], t1 = P.jent[e + 1];
-    for (int t = t0; t < t1; t += 4) {
+    const int t1 = P.jent[e + 1];
+    int t = P.jent[e];
+    auto term = [&](int t, cplx<K> &acc) {
+      const unsigned jt = (unsigned)P.jterms[t];
+      const int term = jt & ((1u << JT_TERM_BITS) - 1);
+      const int q = (jt >> JT_TERM_BITS) & ((1u << JT_PAIR_BITS) - 1);
+      const int ex = jt >> (JT_TERM_BITS + JT_PAIR_BITS);
+      cplx<K> v = w.uj[q];
+      // (a product by 1 is exact in double and double-double)
+      if (K <= 2 || ex != 1) v = Cx::scale_d(v, (double)ex);
+      Cx::mac(acc, coef<K>(P, term), v);
+    };
+    for (; t + 4 <= t1; t += 4) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        if (t + r < t1) {
-          const unsigned jt = (unsigned)P.jterms[t + r];
-          const int term = jt & ((1u << JT_TERM_BITS) - 1);
-          const int q = (jt >> JT_TERM_BITS) & ((1u << JT_PAIR_BITS) - 1);
-          const int ex = jt >> (JT_TERM_BITS + JT_PAIR_BITS);
-          const cplx<K> v = (ex == 1) ? w.uj[q] : Cx::scale_d(w.uj[q], (double)ex);
-          Cx::mac(a[r], coef<K>(P, term), v);
-        }
-      }
+      for (int r = 0; r < 4; ++r) term(t + r, a[r]);
     }
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+      if (t + r < t1) term(t + r, a[r]);
     w.A[e] = Cx::add(Cx::add(a[0], a[1]), Cx::add(a[2], a[3]));
   }
   wsync();
@@ -471,14 +484,18 @@ template <int K> __device__ bool gj_invert_wide(const LProg &__restrict__ P, Pat
 }
 
 // The same inverse for n <= 16 (K <= 2) with the matrix in registers.  Lane (c, g) =
-// (l % 16, l / 16) holds column c of rows g, g+4, g+8, g+12.  Per pivot j:
-// the lanes of column j find the pivot row p among their rows (then across
-// the four of them); the lanes holding row p, row j or column j store those
-// entries to LDS; after one wavefront synchronisation every lane reads the
-// pivot row, the old row j and the pivot column it needs and updates its
-// entries of the swapped, scaled and eliminated matrix in registers.  Each
-// entry gets the operations of the phased version in the same order, so
-// the result is the same bit for bit.  The matrix is stored once at the end.
+// (l % 16, l / 16) holds column c of rows g, g+4, g+8, g+12.  Rows stay where
+// they are: pos is a row's place in the swapped order, and a swap exchanges
+// two places.  Per pivot j: the lanes of column j store it to LDS (col) and
+// find the pivot among their rows (then across the four of them; the largest,
+// the first place among equals); the lanes of the pivot row store it (A); after
+// one wavefront synchronisation every lane reads its entry of the pivot row
+// and its rows' entries of column j and eliminates in registers.  Each entry
+// gets the operations of the phased version in the same order, so the result
+// is the same bit for bit.  The matrix is stored once at the end.
+//   Issue of instructions bounds it (44 of the 490 a pivot took with rows
+// exchanged through selects were FP64 operations): a 12 x 12 inverse with
+// three wavefronts per SIMD took 47.7 k cycles in FP64.
 template <int K> __device__ bool gj_invert(const LProg &__restrict__ P, Path<K> &__restrict__ w) {
   typedef TC<K> Cx;
   const int n = P.n, l = lane_id();
@@ -487,69 +504,83 @@ template <int K> __device__ bool gj_invert(const LProg &__restrict__ P, Path<K> 
   const int c = l & 15, g = l >> 4;
   const bool act = c < n;
   cplx<K> a[4];
+  int pos[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     const int i = g + 4 * s;
+    pos[s] = i;
     a[s] = (act && i < n) ? w.A[i * n + c] : Cx::zero();
   }
-  if (l < n) w.perm[l] = l;
+  wsync();
   for (int j = 0; j < n; ++j) {
     double v = -1.0;
-    int idx = 64;
+    int key = 1 << 16;  // place, row
     if (c == j) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
+        if (4 * s >= n) break;
         const int i = g + 4 * s;
-        if (i >= j && i < n) {
-          double av = absz<K>(a[s]);
-          if (av != av) av = INFINITY;
-          if (av > v) { v = av; idx = i; }
+        if (i < n) {
+          w.col[i] = a[s];
+          if (pos[s] >= j) {
+            double av = absz<K>(a[s]);
+            if (av != av) av = INFINITY;
+            const int k = pos[s] * 16 + i;
+            if (av > v || (av == v && k < key)) { v = av; key = k; }
+          }
         }
       }
     }
     // the four lanes of a column meet (l ^ 16, l ^ 32); column j's result from lane j
-    argmax_stage<16>(v, idx);
-    argmax_stage<32>(v, idx);
-    v = __shfl(v, j, 64);
-    idx = __shfl(idx, j, 64);
+    argmax_stage<16>(v, key);
+    argmax_stage<32>(v, key);
+    key = __builtin_amdgcn_readlane(key, j);
+    v = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), j),
+                         __builtin_amdgcn_readlane(__double2loint(v), j));
     if (!(v > 0.0) || v == INFINITY) return false;
-    const int p = idx;
+    const int row = key & 15, place = key >> 4;
+    if (act && g == (row & 3)) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if ((row >> 2) == s) w.A[c] = a[s];
+    }
+    wsync();  // column j and the pivot row in LDS
+    const cplx<K> inv = Cx::div(Cx::from(1.0, 0.0), w.A[j]);
+    cplx<K> cs[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      const int i = g + 4 * s;
-      if (act && i < n && (i == p || i == j || c == j)) w.A[i * n + c] = a[s];
+      if (4 * s >= n) break;
+      if (g + 4 * s < n) cs[s] = w.col[g + 4 * s];
     }
-    wsync();  // rows p and j and column j of the unswapped matrix in LDS
-    const cplx<K> piv = w.A[p * n + j], cjj = w.A[j * n + j];
-    const cplx<K> inv = Cx::div(Cx::from(1.0, 0.0), piv);
-    if (act) {
-      const cplx<K> rc = w.A[p * n + c], aj = w.A[j * n + c];
-      const cplx<K> r = (c == j) ? inv : Cx::mul(rc, inv);  // scaled pivot row
+    const cplx<K> rc = w.A[act ? c : 0];
+    wsync();  // every read of this pivot before the next pivot's stores
+    if (c == j) {
+      // column j: the negated products with the reciprocal
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        const int i = g + 4 * s;
-        if (i < n) {
-          // entry (i, c) of the swapped matrix: source row p for i = j, j for i = p
-          const cplx<K> cs = (i == j) ? piv : ((i == p) ? cjj : w.A[i * n + j]);
-          const cplx<K> sv = (i == j) ? rc : ((i == p) ? aj : a[s]);
-          cplx<K> nv;
-          if (i == j) nv = r;
-          else if (c == j) nv = Cx::neg(Cx::mul(cs, inv));
-          else {
-            nv = sv;
-            Cx::msub(nv, cs, r);
-          }
-          a[s] = nv;
-        }
+        if (4 * s >= n) break;
+        a[s] = (g + 4 * s == row) ? inv : Cx::neg(Cx::mul(cs[s], inv));
+      }
+    } else {
+      const cplx<K> r = Cx::mul(rc, inv);  // scaled pivot row
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if (4 * s >= n) break;
+        if (g + 4 * s == row) a[s] = r;
+        else Cx::msub(a[s], cs[s], r);
       }
     }
-    if (l == 0 && p != j) { const int t = w.perm[j]; w.perm[j] = w.perm[p]; w.perm[p] = t; }
-    wsync();  // every read of this pivot before the next pivot's stores
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int q = pos[s];
+      pos[s] = q == place ? j : q == j ? place : q;
+    }
   }
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     const int i = g + 4 * s;
-    if (act && i < n) w.A[i * n + c] = a[s];
+    if (act && i < n) w.A[pos[s] * n + c] = a[s];
+    if (c == 0 && i < n) w.perm[pos[s]] = i;
   }
   wsync();
   return true;
@@ -693,47 +724,82 @@ __device__ __forceinline__ void upper_ij(int n, int q, int &i, int &j) {
 template <typename MF>
 __device__ double sigma_max_sq(int n, MF M, LDS double2 *P, LDS double2 *Q, LDS double2 *Y) {
   const int l = lane_id(), nu = n * (n + 1) / 2;
+  // n <= 16: at most 136 upper entries, three per lane, their rows and columns
+  int qi[3], qj[3];
+  double2 q[3];
+  auto store = [&](int r, double sc) {
+    if (l + 64 * r < nu) {
+      const double2 v = make_double2(q[r].x * sc, q[r].y * sc);
+      P[qi[r] * n + qj[r]] = v;
+      P[qj[r] * n + qi[r]] = make_double2(v.x, qi[r] == qj[r] ? v.y : -v.y);
+    }
+  };
   // Hermitian: entries i <= j computed, i > j their conjugates
-  for (int q = l; q < nu; q += 64) {
-    int i, j;
-    upper_ij(n, q, i, j);
-    double2 acc = make_double2(0.0, 0.0);
-    for (int k = 0; k < n; ++k) zcjmac(acc, M(k, i), M(k, j));
-    P[i * n + j] = acc;
-    P[j * n + i] = make_double2(acc.x, i == j ? acc.y : -acc.y);
+  if (n <= 16) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      const int e = l + 64 * r;
+      qi[r] = qj[r] = 0;
+      q[r] = make_double2(0.0, 0.0);
+      if (e < nu) {
+        upper_ij(n, e, qi[r], qj[r]);
+        for (int k = 0; k < n; ++k) zcjmac(q[r], M(k, qi[r]), M(k, qj[r]));
+        P[qi[r] * n + qj[r]] = q[r];
+        P[qj[r] * n + qi[r]] = make_double2(q[r].x, qi[r] == qj[r] ? q[r].y : -q[r].y);
+      }
+    }
+  } else {
+    for (int e = l; e < nu; e += 64) {
+      int i, j;
+      upper_ij(n, e, i, j);
+      double2 acc = make_double2(0.0, 0.0);
+      for (int k = 0; k < n; ++k) zcjmac(acc, M(k, i), M(k, j));
+      P[i * n + j] = acc;
+      P[j * n + i] = make_double2(acc.x, i == j ? acc.y : -acc.y);
+    }
   }
   wsync();
   double tr = 0.0;
   for (int i = 0; i < n; ++i) tr = tr + P[i * n + i].x;
   if (tr != tr) return tr;
   if (!(tr > 0.0)) return 0.0;
-  // P holds the unscaled power; its scaled entries (x*sc) are formed where
-  // read, with the roundings of the oracle's scaled copy
+  // n <= 16: the lanes scale their entries of P by 1 / trace where they keep
+  // them.  Beyond that P holds the unscaled power, whose scaled entries (x*sc)
+  // are formed where read, with the same roundings.
   double sc = 1.0 / tr;
-  for (int s = 0; s < 6; ++s) {
-    auto sp = [&](int e) { const double2 v = P[e]; return make_double2(v.x * sc, v.y * sc); };
-    if (n <= 16) {
-      // at most 136 upper entries: three per lane
-      double2 q[3];
-      int qi[3], qj[3];
+  if (n <= 16) {
+    for (int s = 0; s < 6; ++s) {
+      wsync();  // every lane has the trace
+#pragma unroll
+      for (int r = 0; r < 3; ++r) store(r, sc);
+      wsync();
 #pragma unroll
       for (int r = 0; r < 3; ++r) {
-        const int e = l + 64 * r;
-        q[r] = make_double2(0.0, 0.0);
-        qi[r] = qj[r] = 0;
-        if (e < nu) {
-          upper_ij(n, e, qi[r], qj[r]);
-          for (int k = 0; k < n; ++k) zmac(q[r], sp(qi[r] * n + k), sp(k * n + qj[r]));
+        if (64 * r >= nu) break;
+        double2 acc = make_double2(0.0, 0.0);
+        if (l + 64 * r < nu) {
+          const LDS double2 *x = P + qi[r] * n, *y = P + qj[r];
+          for (int k = 0; k < n; ++k, ++x, y += n) zmac(acc, *x, *y);
         }
+        q[r] = acc;
       }
       wsync();
 #pragma unroll
       for (int r = 0; r < 3; ++r)
-        if (l + 64 * r < nu) {
-          P[qi[r] * n + qj[r]] = q[r];
-          P[qj[r] * n + qi[r]] = make_double2(q[r].x, qi[r] == qj[r] ? q[r].y : -q[r].y);
-        }
-    } else {
+        if (l + 64 * r < nu && qi[r] == qj[r]) P[qi[r] * n + qi[r]] = q[r];
+      wsync();
+      tr = 0.0;
+      for (int i = 0; i < n; ++i) tr = tr + P[i * n + i].x;
+      sc = 1.0 / tr;
+    }
+    wsync();
+#pragma unroll
+    for (int r = 0; r < 3; ++r) store(r, sc);
+    wsync();
+    sc = 1.0;
+  } else {
+    for (int s = 0; s < 6; ++s) {
+      auto sp = [&](int e) { const double2 v = P[e]; return make_double2(v.x * sc, v.y * sc); };
       for (int e = l; e < nu; e += 64) {
         int i, j;
         upper_ij(n, e, i, j);
@@ -744,11 +810,11 @@ __device__ double sigma_max_sq(int n, MF M, LDS double2 *P, LDS double2 *Q, LDS 
       }
       wsync();
       for (int e = l; e < n * n; e += 64) P[e] = Q[e];
+      wsync();
+      tr = 0.0;
+      for (int i = 0; i < n; ++i) tr = tr + P[i * n + i].x;
+      sc = 1.0 / tr;
     }
-    wsync();
-    tr = 0.0;
-    for (int i = 0; i < n; ++i) tr = tr + P[i * n + i].x;
-    sc = 1.0 / tr;
   }
   int jm = 0;
   double best = P[0].x * sc;
@@ -774,7 +840,7 @@ __device__ double sigma_max_sq(int n, MF M, LDS double2 *P, LDS double2 *Q, LDS 
     den = den + vx * vx + vy * vy;
   }
   wsync();
-  return num / den;
+  return uniform(num / den);
 }
 
 // the mixed residual mean_i |f_i| / (|f|_i + 1) at the point in the order-0
@@ -798,16 +864,26 @@ template <int K> __device__ double mixed_residual(const LProg &__restrict__ P, P
   }
   double acc = 0.0;
   if (l < n * G) {
+    // terms of one monomial (adjacent) add up to gz
     double2 gz = make_double2(0.0, 0.0);
+    const LDS int4 *pairs = reinterpret_cast<const LDS int4 *>(P.pairs);
     const int t1 = P.seg[l + 1];
-    for (int t = P.seg[l]; t < t1; ++t) {
-      const int q = P.tpair[t], m = P.pairs[4 * q + 3], r = P.pairs[4 * q];
-      const double2 cw = zmul(P.tcoef[t], lead<K>(w.W[3 * r]));
-      gz.x = gz.x + cw.x;
-      gz.y = gz.y + cw.y;
-      if (t + 1 == t1 || P.pairs[4 * P.tpair[t + 1] + 3] != m) {
-        acc = acc + zrad(gz.x, gz.y) * rn[m];
-        gz = make_double2(0.0, 0.0);
+    int t = P.seg[l];
+    if (t < t1) {
+      int4 pr = pairs[P.tpair[t]];
+      for (;;) {
+        const double2 cw = zmul(P.tcoef[t], lead<K>(w.W[3 * pr.x]));
+        gz.x = gz.x + cw.x;
+        gz.y = gz.y + cw.y;
+        const int m = pr.w;
+        ++t;
+        const bool end = t >= t1;
+        if (!end) pr = pairs[P.tpair[t]];
+        if (end || pr.w != m) {
+          acc = acc + zrad(gz.x, gz.y) * rn[m];
+          gz = make_double2(0.0, 0.0);
+        }
+        if (end) break;
       }
     }
   }
@@ -817,13 +893,16 @@ template <int K> __device__ double mixed_residual(const LProg &__restrict__ P, P
   if (G > 8) acc = acc + bfly<8>(acc);
   if (G > 16) acc = acc + bfly<16>(acc);
   if (G > 32) acc = acc + bfly<32>(acc);
-  if (l < n * G && (l % G) == 0) mr[l / G] = acc;
+  // the quotients in the lanes of the equations, then their sum in order
+  if (l < n * G && (l % G) == 0) {
+    const cplx<K> f = w.rhs[l / G];
+    mr[l / G] = zrad(R<K>::hi(f.re), R<K>::hi(f.im)) / (acc + 1.0);
+  }
   wsync();
   double mix = 0.0;
-  for (int i = 0; i < n; ++i)
-    mix = mix + zrad(R<K>::hi(w.rhs[i].re), R<K>::hi(w.rhs[i].im)) / (mr[i] + 1.0);
+  for (int i = 0; i < n; ++i) mix = mix + mr[i];
   wsync();
-  return mix / (double)n;
+  return uniform(mix / (double)n);
 }
 
 // sum over the equations of sigma_max(Hessian_i)^2 right after the order-0
@@ -1045,8 +1124,8 @@ __device__ __forceinline__ void fabry_radius(const LProg &__restrict__ P, Path<K
     else if (v < m) m = v;
   }
   wsync();
-  *pfail = fail;
-  *r = m;
+  *pfail = uniform((int)fail) != 0;
+  *r = uniform(m);
 }
 
 // the point's value, Jacobian (inverted), Hessian sum, and the Taylor
@@ -1106,7 +1185,7 @@ template <int K> __device__ int mlp_choose(const Ctl &ctl, Path<K> &w, const dou
     v += bfly<32>(v);
     if (v + b3[c] >= ctl.thresh) best = c;
   }
-  return best;
+  return uniform(best);
 }
 
 // [L/2] Pade coefficients of one component's series c[0..L+2] in place
@@ -1259,7 +1338,7 @@ __global__ void __launch_bounds__(64 * MW) track_kernel(DevProgram G, const Para
   for (;;) {
     int path = 0;
     if (l == 0) path = atomicAdd(counter, 1);
-    path = __shfl(path, 0, 64);
+    path = uniform(path);
     if (path >= npaths) break;
     double t = 0.0, dxl = 0.0, hprev = par.maxstep;
     double dxh[4] = {1.0, 1.0, 1.0, 1.0};
@@ -1326,7 +1405,7 @@ __global__ void __launch_bounds__(64 * MW) track_kernel(DevProgram G, const Para
       wsync();
       double nrm = 0.0;
       for (int j = 0; j < n; ++j) nrm = nrm + mr[j].x * mr[j].x + mr[j].y * mr[j].y;
-      nrm = sqrt(nrm);
+      nrm = uniform(sqrt(nrm));
       wsync();
       // ---- curvature step: sigma_min(J) = 1 / sigma_max(J^{-1}) ----
       double step;
@@ -1456,7 +1535,7 @@ __global__ void __launch_bounds__(64 * REFINE_MAX_WAVES) refine_kernel(DevProgra
   for (;;) {
     int path = 0;
     if (l == 0) path = atomicAdd(counter, 1);
-    path = __shfl(path, 0, 64);
+    path = uniform(path);
     if (path >= npaths) break;
     load_point<K>(P, w, xin, KS, npaths, path);
     if (only && only[path] != ST_SUCCESS) {
@@ -1522,7 +1601,7 @@ __global__ void __launch_bounds__(64 * REFINE_MAX_WAVES) endgame_kernel(DevProgr
   for (;;) {
     int path = 0;
     if (l == 0) path = atomicAdd(counter, 1);
-    path = __shfl(path, 0, 64);
+    path = uniform(path);
     if (path >= npaths) break;
     load_point<K>(P, w, x, KS, npaths, path);
     const double t = tend[path], dist = 1.0 - t;
@@ -1647,6 +1726,11 @@ int geometry(const DevProgram &P, int K, int max_waves, int kmax, int npaths, in
   int wv = (int)((cap - prog) / pb);
   if (wv > max_waves) wv = max_waves;
   if (wv > kmax) wv = kmax;
+  // fewer paths than the wavefronts of all compute units: as many units as
+  // possible with fewer wavefronts each (1024 double-double paths on 128 units
+  // with eight wavefronts kept their vector units 96 % busy, the other 128 idle)
+  const int spread = (int)((npaths + (long)ncu - 1) / ncu);
+  if (wv > spread) wv = spread < 1 ? 1 : spread;
   const size_t bytes = prog + (size_t)wv * pb;
   long per_cu = (long)(LDS_PER_CU / bytes);
   if (per_cu < 1) per_cu = 1;
