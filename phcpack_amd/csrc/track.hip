@@ -288,6 +288,21 @@ template <int K> __device__ __forceinline__ cplx<K> coef(const LProg &P, int t) 
   return C<K>::from(c.x, c.y);
 }
 
+// acc += c v for a term's coefficient, whose limbs beyond the first are zero:
+// the products of a K-limb number and a double, which have the bits of the
+// K-limb products with (c, 0, ...) and half of their operations at K = 4
+template <int K> __device__ __forceinline__ void mac_coef(cplx<K> &z, const LProg &P, int t, const cplx<K> &v) {
+  if constexpr (K == 1) {
+    TC<K>::mac(z, coef<K>(P, t), v);
+  } else {
+    const double2 c = P.tcoef[t];
+    z.re = md::add(z.re, md::mul_d(v.re, c.x));
+    z.re = md::sub(z.re, md::mul_d(v.im, c.y));
+    z.im = md::add(z.im, md::mul_d(v.re, c.y));
+    z.im = md::add(z.im, md::mul_d(v.im, c.x));
+  }
+}
+
 template <int K> __device__ __forceinline__ cplx<K> load_weight(const LProg &P, int j) {
   cplx<K> z;
   z.re = R<K>::load(P.weights, 3 * P.ncomp, j);
@@ -382,14 +397,14 @@ template <int K> __device__ void residual(const LProg &__restrict__ P, Path<K> &
     const int t1 = P.seg[l + 1];
     int t = P.seg[l];
     for (; t + 4 <= t1; t += 4) {
-      Cx::mac(a0, coef<K>(P, t), w.u[P.tpair[t]]);
-      Cx::mac(a1, coef<K>(P, t + 1), w.u[P.tpair[t + 1]]);
-      Cx::mac(a2, coef<K>(P, t + 2), w.u[P.tpair[t + 2]]);
-      Cx::mac(a3, coef<K>(P, t + 3), w.u[P.tpair[t + 3]]);
+      mac_coef<K>(a0, P, t, w.u[P.tpair[t]]);
+      mac_coef<K>(a1, P, t + 1, w.u[P.tpair[t + 1]]);
+      mac_coef<K>(a2, P, t + 2, w.u[P.tpair[t + 2]]);
+      mac_coef<K>(a3, P, t + 3, w.u[P.tpair[t + 3]]);
     }
-    if (t < t1) Cx::mac(a0, coef<K>(P, t), w.u[P.tpair[t]]);
-    if (t + 1 < t1) Cx::mac(a1, coef<K>(P, t + 1), w.u[P.tpair[t + 1]]);
-    if (t + 2 < t1) Cx::mac(a2, coef<K>(P, t + 2), w.u[P.tpair[t + 2]]);
+    if (t < t1) mac_coef<K>(a0, P, t, w.u[P.tpair[t]]);
+    if (t + 1 < t1) mac_coef<K>(a1, P, t + 1, w.u[P.tpair[t + 1]]);
+    if (t + 2 < t1) mac_coef<K>(a2, P, t + 2, w.u[P.tpair[t + 2]]);
     acc = Cx::add(Cx::add(a0, a1), Cx::add(a2, a3));
   }
   acc = group_sum<K>(acc, P.G);
@@ -419,7 +434,7 @@ template <int K> __device__ void jacobian(const LProg &__restrict__ P, Path<K> &
       cplx<K> v = w.uj[q];
       // (a product by 1 is exact in double and double-double)
       if (K <= 2 || ex != 1) v = Cx::scale_d(v, (double)ex);
-      Cx::mac(acc, coef<K>(P, term), v);
+      mac_coef<K>(acc, P, term, v);
     };
     for (; t + 4 <= t1; t += 4) {
 #pragma unroll
@@ -431,6 +446,67 @@ template <int K> __device__ void jacobian(const LProg &__restrict__ P, Path<K> &
     w.A[e] = Cx::add(Cx::add(a[0], a[1]), Cx::add(a[2], a[3]));
   }
   wsync();
+}
+
+// x - y (minus) or x + y; the subtraction as the addition of the negated number
+template <class T> __device__ __forceinline__ T add_or_sub(const T &x, const T &y, bool minus) {
+  T z = y;
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(T) / sizeof(double); ++i) z.x[i] = minus ? -y.x[i] : y.x[i];
+  return md::add(x, z);
+}
+
+// Pivot j of the inverse in quad-double, column j in col: the reciprocal of
+// the pivot, the scaled pivot row and the elimination, a lane per real or
+// imaginary part, each with the operations of C<K>::div, mul and msub.  One
+// lane per number ran the two quotients of the reciprocal one after another on
+// every lane, a third of a pivot's operations.
+template <int K> __device__ __forceinline__ void gj_eliminate_parts(int n, int j, Path<K> &__restrict__ w) {
+  typedef typename RealT<K>::type T;
+  const int l = lane_id(), part = l & 1;
+  const bool im = part == 1;
+  cplx<K> inv;
+  {
+    const cplx<K> b = w.col[j];
+    const T den = md::add(md::mul(b.re, b.re), md::mul(b.im, b.im));
+    // re: 1 b.re + 0 b.im, im: 0 b.re - 1 b.im (the numerator of C<K>::div)
+    const T num = add_or_sub(md::mul_d(b.re, im ? 0.0 : 1.0), md::mul_d(b.im, im ? 1.0 : 0.0), im);
+    const T own = md::div(num, den);
+    T other;
+#pragma unroll
+    for (int i = 0; i < K; ++i) other.x[i] = bfly<1>(own.x[i]);
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      inv.re.x[i] = im ? other.x[i] : own.x[i];
+      inv.im.x[i] = im ? own.x[i] : other.x[i];
+    }
+  }
+  auto part_of = [&](int e) -> LDS T & { return *((LDS T *)(w.A + e) + part); };
+  for (int t = l; t < 2 * n; t += 64) {
+    const int e = j * n + (t >> 1);
+    if ((t >> 1) == j) {
+#pragma unroll
+      for (int i = 0; i < K; ++i) part_of(e).x[i] = im ? inv.im.x[i] : inv.re.x[i];
+    } else {
+      const cplx<K> x = w.A[e];
+      part_of(e) = add_or_sub(md::mul(im ? x.im : x.re, inv.re), md::mul(im ? x.re : x.im, inv.im), !im);
+    }
+  }
+  wsync();
+  for (int t = l; t < 2 * n * n; t += 64) {
+    const int e = t >> 1, i = e / n, c = e - i * n;
+    if (i == j) continue;
+    const cplx<K> x = w.col[i];
+    if (c == j) {
+      part_of(e) = md::neg(add_or_sub(md::mul(im ? x.im : x.re, inv.re), md::mul(im ? x.re : x.im, inv.im), !im));
+    } else {
+      // re: - x.re y.re + x.im y.im, im: - x.im y.re - x.re y.im
+      const cplx<K> y = w.A[j * n + c];
+      T z = part_of(e);
+      z = md::sub(z, md::mul(im ? x.im : x.re, y.re));
+      part_of(e) = add_or_sub(z, md::mul(im ? x.re : x.im, y.im), im);
+    }
+  }
 }
 
 // In-place Gauss-Jordan inverse with partial pivoting: A := (P A)^{-1}
@@ -469,14 +545,18 @@ template <int K> __device__ bool gj_invert_wide(const LProg &__restrict__ P, Pat
     }
     if (l < n) w.col[l] = w.A[l * n + j];
     wsync();
-    const cplx<K> inv = Cx::div(Cx::from(1.0, 0.0), w.col[j]);
-    for (int c = l; c < n; c += 64) w.A[j * n + c] = (c == j) ? inv : Cx::mul(w.A[j * n + c], inv);
-    wsync();
-    for (int e = l; e < n * n; e += 64) {
-      const int i = e / n, c = e - i * n;
-      if (i == j) continue;
-      if (c == j) w.A[e] = Cx::neg(Cx::mul(w.col[i], inv));
-      else Cx::msub(w.A[e], w.col[i], w.A[j * n + c]);
+    if constexpr (K >= 4) {
+      gj_eliminate_parts<K>(n, j, w);
+    } else {
+      const cplx<K> inv = Cx::div(Cx::from(1.0, 0.0), w.col[j]);
+      for (int c = l; c < n; c += 64) w.A[j * n + c] = (c == j) ? inv : Cx::mul(w.A[j * n + c], inv);
+      wsync();
+      for (int e = l; e < n * n; e += 64) {
+        const int i = e / n, c = e - i * n;
+        if (i == j) continue;
+        if (c == j) w.A[e] = Cx::neg(Cx::mul(w.col[i], inv));
+        else Cx::msub(w.A[e], w.col[i], w.A[j * n + c]);
+      }
     }
     wsync();
   }
@@ -513,14 +593,16 @@ template <int K> __device__ bool gj_invert(const LProg &__restrict__ P, Path<K> 
   }
   wsync();
   for (int j = 0; j < n; ++j) {
+    // (the compiler would copy the loop for every number of row groups)
+    int nr = uniform(n);
+    asm volatile("" : "+s"(nr));
     double v = -1.0;
     int key = 1 << 16;  // place, row
     if (c == j) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        if (4 * s >= n) break;
         const int i = g + 4 * s;
-        if (i < n) {
+        if (i < nr) {
           w.col[i] = a[s];
           if (pos[s] >= j) {
             double av = absz<K>(a[s]);
@@ -549,8 +631,7 @@ template <int K> __device__ bool gj_invert(const LProg &__restrict__ P, Path<K> 
     cplx<K> cs[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      if (4 * s >= n) break;
-      if (g + 4 * s < n) cs[s] = w.col[g + 4 * s];
+      if (g + 4 * s < nr) cs[s] = w.col[g + 4 * s];
     }
     const cplx<K> rc = w.A[act ? c : 0];
     wsync();  // every read of this pivot before the next pivot's stores
@@ -558,16 +639,16 @@ template <int K> __device__ bool gj_invert(const LProg &__restrict__ P, Path<K> 
       // column j: the negated products with the reciprocal
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        if (4 * s >= n) break;
-        a[s] = (g + 4 * s == row) ? inv : Cx::neg(Cx::mul(cs[s], inv));
+        if (4 * s < nr) a[s] = (g + 4 * s == row) ? inv : Cx::neg(Cx::mul(cs[s], inv));
       }
     } else {
       const cplx<K> r = Cx::mul(rc, inv);  // scaled pivot row
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        if (4 * s >= n) break;
-        if (g + 4 * s == row) a[s] = r;
-        else Cx::msub(a[s], cs[s], r);
+        if (4 * s < nr) {
+          if (g + 4 * s == row) a[s] = r;
+          else Cx::msub(a[s], cs[s], r);
+        }
       }
     }
 #pragma unroll
@@ -957,11 +1038,10 @@ __device__ int lu_newton_steps(const LProg &__restrict__ P, Path<K> &__restrict_
   for (int k = 1; k <= maxit + 1; ++k) {
     ++*count;
     if (k == 1 && !evaluated) {
-      eval_point<K>(P, w, true);
+      eval_point<K>(P, w, false);
       ++*nfirst;
-    } else {
-      jacobian<K>(P, w);
     }
+    jacobian<K>(P, w);
     if (!gj_invert<K>(P, w)) return -1;
     const cplx<K> dx = apply_inverse<K>(P, w);
     double mdx = 0.0;
@@ -1356,7 +1436,15 @@ __global__ void __launch_bounds__(64 * MW) track_kernel(DevProgram G, const Para
     dxh[0] = dxh[1] = dxh[2] = dxh[3] = 1.0;
     st = ST_RUNNING; steps = 0; rej = 0; rejprev = 0;
     load_point<K>(P, w, start, KS, npaths, path);
-    while (st == ST_RUNNING && t < 1.0) {
+    // the steps up to t = 1, then the endpoint Newton: one loop, so that the
+    // corrector's code is there once (the kernel runs out of a 64 KB
+    // instruction cache shared by two compute units)
+    for (;;) {
+      const bool ending = !(t < 1.0);
+      bool evaluated = false;
+      double step = 0.0, tn = 1.0;
+      int pnum = 0, rej0 = rej, nnewt0 = nnewt;
+      if (!ending) {
       // ---- predictor: Taylor series of x(t+s) ----
       set_weights<K>(P, w, t);
       ++npred;
@@ -1395,8 +1483,9 @@ __global__ void __launch_bounds__(64 * MW) track_kernel(DevProgram G, const Para
       }
       const double pole = pfail ? par.maxstep : par.pbeta * r;
       // the [L/PD] predictor of a series of Dk coefficients
-      const int pnum = par.pnum - (D - Dk);
-      const int rej0 = rej, nnewt0 = nnewt;
+      pnum = par.pnum - (D - Dk);
+      rej0 = rej;
+      nnewt0 = nnewt;
       // ---- predictor coefficients and their error estimates ----
       if (l < n) {
         w.x0[l] = w.slots[l * D];
@@ -1408,7 +1497,6 @@ __global__ void __launch_bounds__(64 * MW) track_kernel(DevProgram G, const Para
       nrm = uniform(sqrt(nrm));
       wsync();
       // ---- curvature step: sigma_min(J) = 1 / sigma_max(J^{-1}) ----
-      double step;
       {
         const double lam = sigma_max_sq(
             n, [&](int a, int b) { return lead<K>(w.A[a * n + b]); },
@@ -1428,11 +1516,9 @@ __global__ void __launch_bounds__(64 * MW) track_kernel(DevProgram G, const Para
         if (ctl.pcap > 0.0 && !pfail && r > 0.0) step = fmin(step, ctl.pcap * r);
       }
       // ---- Bounded_Update (three_way_minima.adb:96-109) ----
-      double tn;
       if (t + step >= 1.0 - par.minstep) { step = 1.0 - t; tn = 1.0; }
       else tn = t + step;
       // ---- Predictor_Feedback (standard_predictor_convolutions.adb:958-993) ----
-      bool evaluated = false;
       for (;;) {
         if (l < n) w.slots[l * D] = pade_value<K, PD>(w.slots + l * D, pnum, w.x0[l], step);
         wsync();
@@ -1446,11 +1532,17 @@ __global__ void __launch_bounds__(64 * MW) track_kernel(DevProgram G, const Para
         tn = t + step;
         if (step < par.minstep) break;
       }
+      }
       // ---- corrector, halving the step on failure ----
       for (;;) {
         if (!evaluated) set_weights<K>(P, w, tn);
-        const int nr =
-            lu_newton_steps<K>(P, w, par.corsteps, par.tolcor, evaluated, &dxl, &nnewt, &nfirst, dxh);
+        const int nr = lu_newton_steps<K>(P, w, ending ? par.endsteps : par.corsteps,
+                                          ending ? par.tolend : par.tolcor, evaluated, &dxl, &nnewt,
+                                          &nfirst, dxh);
+        if (ending) {
+          st = (nr < 0) ? ST_SINGULAR : ST_SUCCESS;
+          break;
+        }
         ++ncorr;
         if (nr < 0) {
           st = ST_SINGULAR;
@@ -1472,6 +1564,7 @@ __global__ void __launch_bounds__(64 * MW) track_kernel(DevProgram G, const Para
         wsync();
         evaluated = false;
       }
+      if (ending) break;
       rejprev = rej - rej0;
       if (ctl.mode == 2 && nlog < ctl.cap) {
         // accepted at the first attempt: the Newton iterations it took (>= 1)
@@ -1483,12 +1576,6 @@ __global__ void __launch_bounds__(64 * MW) track_kernel(DevProgram G, const Para
       ++steps;
       if (max_abs_x<K>(P, w) > par.divergence) { st = ST_DIVERGED; break; }
       if (steps >= par.maxsteps && t < 1.0) { st = ST_MAXSTEPS; break; }
-    }
-    if (st == ST_RUNNING) {
-      set_weights<K>(P, w, 1.0);
-      const int nr =
-          lu_newton_steps<K>(P, w, par.endsteps, par.tolend, false, &dxl, &nnewt, &nfirst, nullptr);
-      st = (nr < 0) ? ST_SINGULAR : ST_SUCCESS;
     }
     if (!(pmode == 1 && st != ST_SUCCESS && t < ctl.retry)) break;
     }
