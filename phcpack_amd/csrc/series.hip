@@ -48,6 +48,7 @@ template <int K> struct Num<K, false> {
   __device__ static void inc(V &c, const V &a) { c = md::add(c, a); }
   __device__ static V zero() { return R<K>::zero(); }
   __device__ static V pick(bool c, const V &a, const V &b) { return pick_real(c, a, b); }
+  __device__ static V pick_v(bool c, const V &a, const V &b) { return pick_real(c, a, b); }
 };
 template <int K> struct Num<K, true> {
   typedef cplx<K> V;
@@ -60,6 +61,12 @@ template <int K> struct Num<K, true> {
   __device__ static void inc(V &c, const V &a) { c = C<K>::add(c, a); }
   __device__ static V zero() { return C<K>::zero(); }
   template <class T> __device__ static T pick(bool c, const T &a, const T &b) { return pick_real(c, a, b); }
+  __device__ static V pick_v(bool c, const V &a, const V &b) {
+    V v;
+    v.re = pick_real(c, a.re, b.re);
+    v.im = pick_real(c, a.im, b.im);
+    return v;
+  }
 };
 
 // ----------------------------------------------------------- elementwise --
@@ -90,21 +97,6 @@ __device__ typename N::V coef_product(const double *x, size_t sx, size_t xo, con
   return acc;
 }
 
-// z[b] = x[b]*y[b] for b < nbatch; arrays [P][nbatch][D]
-template <int K, bool CPLX>
-__global__ void __launch_bounds__(256) product_kernel(int D, int nbatch, const double *x, const double *y, double *z) {
-  typedef Num<K, CPLX> N;
-  const size_t s = (size_t)nbatch * D;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < s;
-       t += (size_t)gridDim.x * blockDim.x) {
-    const size_t b = t / D;
-    const int k = (int)(t % D);
-    N::store(z, s, t, coef_product<N>(x, s, b * D, y, s, b * D, k));
-  }
-}
-
-// ------------------------------------------------ polynomial eval / diff --
-
 // acc = x*y when first, else acc + x*y, each in the order of N::mul and N::mac
 template <class N>
 __device__ __forceinline__ void mac_or_mul(typename N::V &acc, bool first, const typename N::V &x,
@@ -122,25 +114,80 @@ __device__ __forceinline__ void mac_or_mul(typename N::V &acc, bool first, const
 }
 
 // Two truncated products at once by the D lanes of a group: lane k forms
-// coefficient k of x1*y1, then coefficient D-1-k of x2*y2 (when two), so that
-// every lane does D + 1 multiply-adds, where one lane per coefficient of one
-// product leaves half of the lanes idle on average.  The terms of a
-// coefficient keep the order of coef_product.  x1, ...: offsets of the rows
-// in the planar array p (plane stride s).
+// coefficient k of x1*y1, then coefficient D-1-k of x2*y2 (no second product:
+// any rows, the result unused), D + 1 multiply-adds on every lane, where one
+// lane per coefficient of one product leaves half of the lanes idle on
+// average.  The terms of a coefficient keep the order of coef_product.  In
+// double-double a sum starts from zero, to which the first product (never -0 in
+// its head) is added without a change.  x1, ...: offsets of the rows in p, numbers with their
+// limbs side by side.
 template <class N>
-__device__ __forceinline__ void product_pair(const double *p, size_t s, int x1, int y1, int x2, int y2,
-                                             int D, int k, bool two, typename N::V &r1,
-                                             typename N::V &r2) {
-  typename N::V acc = N::zero();
-  const int T = two ? D + 1 : k + 1;
-  for (int it = 0; it < T; ++it) {
-    const bool second = it > k;
-    const int xo = second ? x2 + (it - k - 1) : x1 + it, yo = second ? y2 + (D - it) : y1 + (k - it);
-    mac_or_mul<N>(acc, it == 0 || it == k + 1, N::load(p, s, xo), N::load(p, s, yo));
-    if (it == k) r1 = acc;
+__device__ __forceinline__ void product_pair(const double *p, int x1, int y1, int x2, int y2, int D, int k,
+                                             typename N::V &r1, typename N::V &r2) {
+  constexpr int P = N::P, U = P <= 4 ? 2 : 1;
+  constexpr bool from_zero = (N::CX ? P / 2 : P) == 2;
+  const double *px = p + x1 * P, *py = p + (y1 + k) * P, *const px2 = p + x2 * P,
+               *const py2 = p + (y2 + D - 1 - k) * P;
+  typename N::V acc = N::zero(), turned = N::zero();
+  bool first = true;
+#pragma unroll U
+  for (int it = 0; it <= D; ++it) {
+    const typename N::V x = N::load(px, 1, 0), y = N::load(py, 1, 0);
+    if constexpr (from_zero) N::mac(acc, x, y);
+    else mac_or_mul<N>(acc, first, x, y);
+    const bool turn = it == k;
+    turned = N::pick_v(turn, acc, turned);
+    if constexpr (from_zero) acc = N::pick_v(turn, N::zero(), acc);
+    first = turn;
+    px = turn ? px2 : px + P;
+    py = turn ? py2 : py - P;
   }
+  r1 = turned;
   r2 = acc;
 }
+
+// z[b] = x[b]*y[b] for b < nbatch; arrays [P][nbatch][D]
+template <int K, bool CPLX>
+__global__ void __launch_bounds__(256) product_kernel(int D, int nbatch, const double *x, const double *y, double *z) {
+  typedef Num<K, CPLX> N;
+  const size_t s = (size_t)nbatch * D;
+  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < s;
+       t += (size_t)gridDim.x * blockDim.x) {
+    const size_t b = t / D;
+    const int k = (int)(t % D);
+    N::store(z, s, t, coef_product<N>(x, s, b * D, y, s, b * D, k));
+  }
+}
+
+// The same for many products: D lanes take two of them, staged through LDS (4
+// rows of D numbers), in blocks of gpb groups.  4096 complex quad-double
+// products of degree 31: 155 us with a lane per coefficient, whose loads are
+// from global memory and whose lanes idle half of the time, 85 us here.
+template <int K, bool CPLX>
+__global__ void __launch_bounds__(256) product_pair_kernel(int D, int nbatch, const double *__restrict__ x,
+                                       const double *__restrict__ y, double *__restrict__ z, int gpb) {
+  typedef Num<K, CPLX> N;
+  extern __shared__ __align__(16) double lds[];
+  const size_t s = (size_t)nbatch * D;
+  const int grp = threadIdx.x / D, k = threadIdx.x % D;
+  const size_t b = 2 * ((size_t)blockIdx.x * gpb + grp);
+  const bool on = grp < gpb && b < (size_t)nbatch, two = on && b + 1 < (size_t)nbatch;
+  double *w = lds + (size_t)grp * 4 * D * N::P;
+  if (on) {
+    N::store(w + k * N::P, 1, 0, N::load(x, s, b * D + k));
+    N::store(w + (D + k) * N::P, 1, 0, N::load(y, s, b * D + k));
+    N::store(w + (2 * D + k) * N::P, 1, 0, two ? N::load(x, s, b * D + D + k) : N::zero());
+    N::store(w + (3 * D + k) * N::P, 1, 0, two ? N::load(y, s, b * D + D + k) : N::zero());
+  }
+  __syncthreads();
+  if (!on) return;
+  typename N::V r1, r2;
+  product_pair<N>(w, 0, D, 2 * D, 3 * D, D, k, r1, r2);
+  N::store(z, s, b * D + k, r1);
+  if (two) N::store(z, s, b * D + 2 * D - 1 - k, r2);
+}
+
+// ------------------------------------------------ polynomial eval / diff --
 
 // The contributions of every monomial at every instance: monomial i's value
 // and its derivatives with respect to idx[idxptr[i]..], in slots idxptr[i]+i
@@ -155,7 +202,7 @@ __device__ __forceinline__ void product_pair(const double *p, size_t s, int x1, 
 // global memory, took 16.4 ms for one double-double polynomial of 560
 // monomials at degree 31 (29 us a monomial, two of the chip's wavefronts
 // busy); monomials are independent, and only the sums over them have an
-// order, which poly_sum_kernel keeps: 75 us for the two kernels.  1021
+// order, which poly_sum_kernel keeps: 74 us for the two kernels.  1021
 // instances of 10 complex quad-double monomials of 4 variables at degree 15:
 // 3.59 -> 0.91 ms (15 TFLOP/s of FP64 operations; the FP64 pipes, about 40
 // TFLOP/s without fused multiply-adds, bound it).
@@ -167,7 +214,7 @@ __global__ void __launch_bounds__(256) poly_terms_kernel(int dim, int nbr, int D
                                      double *__restrict__ contrib, size_t sT, double *work, int gpb) {
   typedef Num<K, CPLX> N;
   typedef typename N::V V;
-  extern __shared__ double lds[];
+  extern __shared__ __align__(16) double lds[];
   const int grp = threadIdx.x / D, k = threadIdx.x % D;
   const size_t gid = (size_t)blockIdx.x * gpb + grp;
   const bool on = grp < gpb && gid < (size_t)nbr * nb;
@@ -175,13 +222,14 @@ __global__ void __launch_bounds__(256) poly_terms_kernel(int dim, int nbr, int D
   const int nv = on ? nvr[i] : 0;
   const int *ix = idx + idxptr[i];
   const size_t sX = (size_t)nbatch * dim * D, xb = (size_t)(b0 + b) * dim * D, sC = (size_t)nbr * D;
-  const size_t s = (size_t)rows * D;  // plane stride of the work area
-  double *w = LW ? lds + (size_t)grp * s * N::P : work + gid * s * N::P;
+  // the group's work area: numbers with their limbs side by side
+  double *w = LW ? lds + (size_t)grp * rows * D * N::P : work + gid * rows * D * N::P;
+  auto keep = [&](int row, int q, const V &v) { N::store(w + (row * D + q) * N::P, 1, 0, v); };
   auto slot = [&](int j) { return ((size_t)(idxptr[i] + i + j) * nb + b) * D + k; };
   if (on) {
-    for (int j = 0; j < nv; ++j) N::store(w, s, j * D + k, N::load(input, sX, xb + (size_t)ix[j] * D + k));
+    for (int j = 0; j < nv; ++j) keep(j, k, N::load(input, sX, xb + (size_t)ix[j] * D + k));
     const V c = N::load(cff, sC, (size_t)i * D + k);
-    N::store(w, s, nv * D + k, c);
+    keep(nv, k, c);
     if (nv == 1) N::store(contrib, sT, slot(1), c);
   }
   const int C = nv, F = nv + 1, B = 2 * nv;  // rows: X 0..nv-1, C, F 0..nv-2, B 0..nv-3
@@ -214,12 +262,12 @@ __global__ void __launch_bounds__(256) poly_terms_kernel(int dim, int nbr, int D
     if (x1 >= 0) {
       V r1, r2;
       const bool two = x2 >= 0;
-      product_pair<N>(w, s, x1 * D, y1 * D, x2 * D, y2 * D, D, k, two, r1, r2);
-      if (d1 >= 0) N::store(w, s, d1 * D + k, r1);
+      product_pair<N>(w, x1 * D, y1 * D, two ? x2 * D : 0, y2 * D, D, k, r1, r2);
+      if (d1 >= 0) keep(d1, k, r1);
       if (s1 >= 0) N::store(contrib, sT, slot(s1), r1);
       if (two) {
         const int k2 = D - 1 - k;
-        if (d2 >= 0) N::store(w, s, d2 * D + k2, r2);
+        if (d2 >= 0) keep(d2, k2, r2);
         if (s2 >= 0) N::store(contrib, sT, slot(s2) + k2 - k, r2);
       }
     }
@@ -296,9 +344,28 @@ int phc_series_product(int K, int cplx, int deg, int nbatch, const double *x, co
   PHC_REQUIRE(deg >= 0 && nbatch >= 0, "phc_series_product: negative size");
   if (nbatch == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
-  const int D = deg + 1, block = 256;
-  const int grid = phc::grid_for((size_t)nbatch * D, block);
-#define PL(KK, CC) hipLaunchKernelGGL((product_kernel<KK, CC>), dim3(grid), dim3(block), 0, st, D, nbatch, x, y, z)
+  const int D = deg + 1, P = cplx ? 2 * K : K;
+  // Pairs of products where the arithmetic outweighs the staging and the four
+  // rows of every group fit LDS, else a coefficient per lane.  One lane against
+  // pairs, us: real double-double, degree 31, 16 products 7.5 / 5.6, 8192 19.7 /
+  // 9.5; quad-double, degree 15, 21.5 / 20.0 and 34.5 / 22.5; but double-double
+  // of degree 8, 128 products 3.4 / 3.6, 8192 4.1 / 3.8 (complex 5.1 / 5.5, 7.7 /
+  // 6.3) and double of degree 15, 8192 products 3.8 / 4.4.
+  const int pblock = D <= 64 ? 64 : (D + 63) / 64 * 64, gpb = pblock / D > 0 ? pblock / D : 1;
+  const size_t lds = sizeof(double) * 4 * P * (size_t)D * gpb;
+  const bool pairs = D <= 256 && lds <= 64 * 1024 &&
+                     (K * D >= 64 || (K > 1 && (size_t)nbatch * D >= 65536));
+  const int block = 256, grid = phc::grid_for((size_t)nbatch * D, block);
+  const size_t ngrp = ((size_t)nbatch + 1) / 2, pgrid = (ngrp + gpb - 1) / gpb;
+  PHC_REQUIRE(!pairs || pgrid < (1u << 31), "phc_series_product: too many products");
+#define PL(KK, CC)                                                                               \
+  do {                                                                                           \
+    if (pairs)                                                                                   \
+      hipLaunchKernelGGL((product_pair_kernel<KK, CC>), dim3(pgrid), dim3(pblock), lds, st, D,   \
+                         nbatch, x, y, z, gpb);                                                  \
+    else                                                                                         \
+      hipLaunchKernelGGL((product_kernel<KK, CC>), dim3(grid), dim3(block), 0, st, D, nbatch, x, y, z); \
+  } while (0)
   if (!cplx) {
     if (K == 1) PL(1, false); else if (K == 2) PL(2, false); else if (K == 4) PL(4, false); else PL(8, false);
   } else {

@@ -57,6 +57,29 @@ def test_product_batch_vs_oracle(K, cplx):
             assert np.array_equal(z[:, b], zb), (K, cplx, deg, b)
 
 
+# both sides of each line of the rule for pairs of products: K*D at 63..64,
+# K = 2 at 65536 coefficients, a row of 256 and 257, the LDS limit (D = 128 at
+# complex octo-double, 129 not), blocks with idle lanes, odd and even batches,
+# and signed zeros in double
+@pytest.mark.parametrize("K,cplx,deg,nb", [(1, 0, 62, 3), (1, 0, 63, 3), (1, 1, 63, 4), (1, 0, 255, 5),
+                                           (1, 0, 256, 5), (2, 0, 30, 2), (2, 1, 31, 1), (2, 1, 0, 65535),
+                                           (2, 1, 8, 7281), (2, 1, 8, 7282), (4, 0, 14, 6), (4, 1, 42, 7),
+                                           (8, 0, 7, 33), (8, 1, 127, 2), (8, 1, 128, 2)])
+def test_product_pairs_vs_oracle(K, cplx, deg, nb):
+    from phcpack_amd.series import product
+    rng = np.random.default_rng(7 * deg + nb)
+    gen = (lambda s: rand_cmd(rng, K, s)) if cplx else (lambda s: rand_md(rng, K, s))
+    x, y = gen((nb, deg + 1)), gen((nb, deg + 1))
+    if K == 1:
+        x[:, :, 0] = -0.0
+    z = product(K, cplx, x, y)
+    for b in range(nb) if nb < 100 else (0, 1, nb // 2, nb - 2, nb - 1):
+        xb, yb = np.ascontiguousarray(x[:, b]), np.ascontiguousarray(y[:, b])
+        zb = np.zeros_like(xb)
+        oracle().osr_product(K, cplx, deg, pd(xb), pd(yb), pd(zb))
+        assert np.array_equal(z[:, b], zb) and np.array_equal(np.signbit(z[:, b]), np.signbit(zb)), b
+
+
 @pytest.mark.parametrize("K", [2, 4, 8])
 @pytest.mark.parametrize("cplx", [0, 1])
 def test_product_golden(K, cplx):
