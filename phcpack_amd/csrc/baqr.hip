@@ -384,12 +384,17 @@ template <int K> __device__ __noinline__ T<K> nl_add(T<K> a, T<K> b) { return ad
 template <int K> __device__ __noinline__ T<K> nl_sub(T<K> a, T<K> b) { return sub(a, b); }
 template <int K> __device__ __noinline__ T<K> nl_mul(T<K> a, T<K> b) { return mul(a, b); }
 template <int K> __device__ __noinline__ T<K> nl_div(T<K> a, T<K> b) { return div(a, b); }
-// md::sqrt<4> (a double-double root, then one Newton correction) with its
-// product, sum and quotient as the calls above
+// K = 4: a double-double root b, then the Newton correction b + (a - b^2) / 2b,
+// whose quotient is of the size of the last two limbs and is formed in
+// double-double (a quad-double quotient, as in md::sqrt<4>, has three times as
+// long a chain and changes the last limb's rounding only)
 template <int K> __device__ __noinline__ T<K> nl_sqrt(T<K> a) {
   if constexpr (K == 4) {
-    const T<K> b = widen_half<4>(md::sqrt(lead_half<4>(a)));
-    return mul_pwr2<4>(nl_div<K>(nl_add<K>(nl_mul<K>(b, b), a), b), 0.5);
+    const auto b = md::sqrt(lead_half<4>(a));
+    const T<K> wb = widen_half<4>(b);
+    const auto r = lead_half<4>(nl_sub<K>(a, nl_mul<K>(wb, wb)));
+    if (b.x[0] == 0.0) return wb;  // a zero pivot
+    return nl_add<K>(wb, widen_half<4>(md::div(md::mul_pwr2(r, 0.5), b)));
   } else {
     return R<K>::sqrt(a);
   }
@@ -429,7 +434,12 @@ constexpr int CW = 256;  // lanes (rows) per workgroup of the panel kernels
 // three launches of 28 + 12 + 9 us a column (1024 x 1024 complex quad-double),
 // each waiting for the previous one's sums.  What bounds the step is the
 // chain of dependent quad-double operations: two roots on two lanes, two
-// divisions, the butterflies of the sums.
+// divisions, the butterflies of the sums.  One launch took 43 us a column; with
+// the root's correction in double-double and the four real products of H inv on
+// four lanes, and the S factor and the tile inverse reading ahead, the 1024 x
+// 1024 solve went from 58.4 to 53.3 ms.  beta and 1/v0 straight from sigma, nrm
+// and r0 (one division fewer) reached 49.7 ms but rounded apart: twice the mean
+// error of 40 x 40 double-double factors.
 //
 //   Workgroup (c, s): column j = colidx + c, rows of split s (CW of them, one
 // per lane, counted from the pivot row).  hpart[s][c]: the partial sums of H
@@ -534,10 +544,16 @@ panel_step_kernel(const double *Pin, double *Pout, size_t pps, int m, int rowoff
       w.re = nl_mul<K>(beta, nl_add<K>(r0g.re, nl_mul<K>(h.re, inv.re)));
       w.im = R<K>::zero();
     } else {
-      const T<K> hre = nl_sub<K>(nl_mul<K>(h.re, inv.re), nl_mul<K>(h.im, inv.im));
-      const T<K> him = nl_add<K>(nl_mul<K>(h.im, inv.re), nl_mul<K>(h.re, inv.im));
-      w.re = nl_mul<K>(beta, nl_add<K>(r0g.re, hre));
-      w.im = nl_mul<K>(beta, nl_sub<K>(him, r0g.im));
+      // real part on lanes with t & 3 < 2, imaginary on the others, a product
+      // of each pair on either lane
+      const bool od = t & 1, im = t & 2;
+      h.re = lane_r<K>(h.re, t & 48);  // few splits: the sum is on lane u = 0 only
+      h.im = lane_r<K>(h.im, t & 48);
+      const T<K> p = nl_mul<K>(od == im ? h.re : h.im, od ? inv.im : inv.re);
+      const T<K> o = bfly_r<1, K>(od && !im ? neg(p) : p);
+      const T<K> wc = nl_mul<K>(beta, nl_add<K>(im ? neg(r0g.im) : r0g.re, nl_add<K>(od && !im ? neg(p) : p, o)));
+      w.re = wc;
+      w.im = bfly_r<2, K>(wc);
     }
     if (t == 0) {
       sflag = szero ? 1 : 0;
@@ -843,26 +859,38 @@ __global__ void __launch_bounds__(64)
 s_factor_kernel(const double *G, size_t gps, const double *Bv, double *S, size_t sps, int szt) {
   const int m = blockIdx.x, l = threadIdx.x;
   constexpr int NJ = 2;  // szt <= 128
-  Z<K> acc[NJ];
+  Z<K> acc[NJ], g[NJ];  // sums, and row k of G, read one row ahead
+  auto row = [&](int k) {
 #pragma unroll
-  for (int q = 0; q < NJ; ++q) acc[q] = C<K>::zero();
+    for (int q = 0; q < NJ; ++q) {
+      const int j = l + 64 * q;
+      if (j > k && j < szt) g[q] = C<K>::load(G, gps, (size_t)k * szt + j);
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < NJ; ++q) acc[q] = g[q] = C<K>::zero();
+  T<K> b = R<K>::load(Bv, szt, m);
+  row(m);
   for (int k = m; k < szt; ++k) {
-    const T<K> b = neg(R<K>::load(Bv, szt, k));
-    const Z<K> a = (k >> 6) ? acc[1] : acc[0];
+    const T<K> nb = neg(b);
+    const Z<K> gk[NJ] = {g[0], g[1]}, a = (k >> 6) ? acc[1] : acc[0];
+    if (k + 1 < szt) {
+      b = R<K>::load(Bv, szt, k + 1);
+      row(k + 1);
+    }
     Z<K> v;
     if (k == m) {
-      v.re = b;
+      v.re = nb;
       v.im = R<K>::zero();
     } else {
-      v.re = mul(b, lane_r<K>(a.re, k & 63));
-      v.im = mul(b, lane_r<K>(a.im, k & 63));
+      v.re = mul(nb, lane_r<K>(a.re, k & 63));
+      v.im = mul(nb, lane_r<K>(a.im, k & 63));
     }
     if (l == (k & 63)) C<K>::store(S, sps, (size_t)m * szt + k, v);
 #pragma unroll
     for (int q = 0; q < NJ; ++q) {
       const int j = l + 64 * q;
-      if (j > k && j < szt)
-        acc[q] = C<K>::add(acc[q], C<K>::mul(v, C<K>::load(G, gps, (size_t)k * szt + j)));
+      if (j > k && j < szt) acc[q] = C<K>::add(acc[q], C<K>::mul(v, gk[q]));
     }
   }
   for (int j = l; j < m; j += 64) C<K>::store(S, sps, (size_t)m * szt + j, C<K>::zero());
@@ -898,8 +926,19 @@ tile_inverse_kernel(const double *U, size_t ups, int dim, int szt, int ntiles, d
   }
   for (int r = l; r < szt; r += 64) C<K>::store(x, 256, r, C<K>::from(r == j ? 1.0 : 0.0, 0.0));
   wave_sync();
+  // the rows of column i of U above the diagonal, read one column ahead
+  Z<K> uc[NR];
+  auto column = [&](int i) {
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+      if (K < 8 && l + 64 * q < i) uc[q] = u(l + 64 * q, i);
+  };
+  column(j);
   for (int i = j; i >= 0; --i) {
-    Z<K> v = C<K>::load(x, 256, i);
+    Z<K> v = C<K>::load(x, 256, i), ui[NR];
+#pragma unroll
+    for (int q = 0; q < NR; ++q) ui[q] = uc[q];
+    column(i - 1);
     if constexpr (K == 8) {
       v = C<K>::div(v, u(i, i));
     } else {
@@ -913,8 +952,16 @@ tile_inverse_kernel(const double *U, size_t ups, int dim, int szt, int ntiles, d
     }
     wave_sync();
     if (l == (i & 63)) C<K>::store(x, 256, i, v);
-    for (int r = l; r < i; r += 64)
-      C<K>::store(x, 256, r, C<K>::sub(C<K>::load(x, 256, r), C<K>::mul(u(r, i), v)));
+    if constexpr (K == 8) {
+      for (int r = l; r < i; r += 64)
+        C<K>::store(x, 256, r, C<K>::sub(C<K>::load(x, 256, r), C<K>::mul(u(r, i), v)));
+    } else {
+#pragma unroll
+      for (int q = 0; q < NR; ++q) {
+        const int r = l + 64 * q;
+        if (r < i) C<K>::store(x, 256, r, C<K>::sub(C<K>::load(x, 256, r), C<K>::mul(ui[q], v)));
+      }
+    }
     wave_sync();
   }
   for (int i = l; i < szt; i += 64) C<K>::store(inv, ips, ib + (size_t)i * szt + j, C<K>::load(x, 256, i));

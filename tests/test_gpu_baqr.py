@@ -249,3 +249,36 @@ def test_qr_by_digit_products(K, shape, real, n1):
     print(f"  K={K} {shape} real={real} n1={n1}: Q {dq / ulps(K):.1f} u, R {dr / ulps(K):.1f} u, "
           f"small R {ds / ulps(K):.1f} u", flush=True)
     assert dq < tol and dr < tol * np.sqrt(m) and ds < tol * np.sqrt(m)
+
+
+# the scalars of a column: a zero pivot, a zero column below it, one of size
+# 2^-20 below it (below 2^-52 the formulas' v0 is zero in double-double); and data near 2^-300 and 2^300, where the same factor Q and
+# the exactly scaled R are expected
+@pytest.mark.parametrize("K", [2, 4])
+@pytest.mark.parametrize("kind", ["zero_pivot", "zero_below", "small_below", "scale"])
+def test_qr_column_scalars(K, kind):
+    from phcpack_amd.baqr import BlockedQR
+    m, n, szt = 40, 24, 8
+    A = rand_cmd(np.random.default_rng(5 * K), K, (m, n))
+    if kind == "zero_pivot":
+        A[:, 0, 0] = 0.0
+    elif kind == "zero_below":
+        A[:, 1:, 0] = 0.0
+    elif kind == "small_below":
+        A[:, 1:, 0] *= 2.0 ** -20
+    Q, R = BlockedQR(K, m, n, szt).factor(A)
+    if kind == "scale":
+        for e in (-300.0, 300.0):
+            Qs, Rs = BlockedQR(K, m, n, szt).factor(A * 2.0 ** e)
+            assert np.array_equal(Qs, Q) and np.array_equal(Rs * 2.0 ** -e, R), e
+    # the oracle divides by zero for a zero pivot in quad-double (its root of 0)
+    # and its v0 = x0 - mu x0 cancels 40 bits in small_below: there the factors
+    # are checked in double, Q^H Q = I and Q R = A, whose errors are a few m eps
+    if kind in ("zero_below", "scale") or (kind == "zero_pivot" and K == 2):
+        tol = QR_UNITS * m * ulps(K)
+        Qo, Ro = oracle_blocked_houseqr(K, A, szt, n // szt)
+        assert np.abs(md_diff(K, Q, Qo)).max() < tol and np.abs(md_diff(K, R, Ro)).max() < tol * np.sqrt(m)
+    Ad, Qd, Rd = (X[0] + 1j * X[K] for X in (A, Q, R))
+    tol = 8 * m * 2.0 ** -52
+    assert np.abs(Qd.conj().T @ Qd - np.eye(m)).max() < tol
+    assert np.abs(Qd @ Rd - Ad).max() < tol * np.sqrt(m)
