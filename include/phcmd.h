@@ -458,7 +458,7 @@ int phc_rowsys_destroy(phc_rowsys *sys);
 int phc_rowsys_lds_bytes(const phc_rowsys *sys, int K, int deg, size_t *bytes);
 
 /* staggered row Newton on nsys systems with the same supports, one
- * wavefront per system: working degrees 0, 1, 2, 4, 7, ... capped at deg,
+ * wavefront per system (up to four when there are few): working degrees 0, 1, 2, 4, 7, ... capped at deg,
  * at most nbsteps steps, stopping when the tail index reaches deg.  Each
  * step evaluates and differentiates the system at the series x, solves the
  * linearized block-Toeplitz system and updates x, as dbl2_row_newton_qrstep

@@ -204,7 +204,7 @@ __global__ void __launch_bounds__(256) product_pair_kernel(int D, int nbatch, co
 // busy); monomials are independent, and only the sums over them have an
 // order, which poly_sum_kernel keeps: 74 us for the two kernels.  1021
 // instances of 10 complex quad-double monomials of 4 variables at degree 15:
-// 3.59 -> 0.91 ms (15 TFLOP/s of FP64 operations; the FP64 pipes, about 40
+// 3.59 -> 0.88 ms (16 TFLOP/s of FP64 operations; the FP64 pipes, about 40
 // TFLOP/s without fused multiply-adds, bound it).
 template <int K, bool CPLX, bool LW>
 __global__ void __launch_bounds__(256) poly_terms_kernel(int dim, int nbr, int D, int nvmax, int rows,
